@@ -44,11 +44,20 @@ namespace {
 
 constexpr int kMaxBasis = 64;  // kspace + 1 <= 64
 constexpr int kTile = 8;       // basis vectors per dot tile
-// row blocks of the fused dot kernels: 2048 keeps 8 waves per CU busy even
-// for a short tile (512 measured 2 % / 4 % slower for the FP64 / FP32
-// solves at 256^3, whose dots were latency-bound; 4096-8192 no better)
+// row blocks of the fused dot kernels at most
 constexpr int kRowBlocks = 2048;
 constexpr int kDotVals = 2 * kTile + 3;  // per tile: Q.y, Q.z, y.y, y.z, z.z
+
+// Row blocks of a dot over n rows (vec of them per lane and step) in ntiles
+// tiles: one step per block until the blocks fill the chip (256 CUs), then
+// up to kDotSteps steps, which pay for the reduction a block ends in.
+inline int dot_row_blocks(int64_t n, int vec, int ntiles)
+{
+  constexpr int64_t kDotSteps = 4;
+  const int64_t one = std::max<int64_t>(1, (n / vec + kBlock - 1) / kBlock);
+  const int64_t fill = std::max(1, 1024 / ntiles);
+  return (int)std::min({one, std::max(fill, one / kDotSteps), (int64_t)kRowBlocks});
+}
 
 __device__ inline double wave_sum(double v)
 {
@@ -77,15 +86,40 @@ __device__ inline void block_reduce_store(double (&acc)[NA],
   }
 }
 
-// out[v] = sum_b partial[b * nv + v] over nb blocks, one workgroup per value,
-// fixed-order tree (reproducible).
+// Sums of 16 values over the 64 lanes of a wave by halving: at each step a
+// lane keeps the half of its values that its lane bit names and adds the
+// partner's share of them, so 15 exchanges leave one value per group of four
+// lanes and two more finish it (96 exchanges with a butterfly per value).
+// Lane 4 k + {0..3} returns the sum of value k.
+__device__ inline double wave_sum16(double (&a)[16])
+{
+  const int lane = threadIdx.x & 63;
+#pragma unroll
+  for (int h = 8; h >= 1; h >>= 1) {
+    const int o = 4 * h;  // lane bit 5, 4, 3, 2
+    const bool up = lane & o;
+#pragma unroll
+    for (int i = 0; i < h; ++i) {
+      const double keep = up ? a[h + i] : a[i];
+      const double send = up ? a[i] : a[h + i];
+      a[i] = keep + __shfl_xor(send, o);
+    }
+  }
+  double v = a[0];
+  v += __shfl_xor(v, 2);
+  v += __shfl_xor(v, 1);
+  return v;
+}
+
+// out[v] = sum_b partial[v * nb + b], one workgroup per value, fixed-order
+// tree (reproducible).
 __global__ __launch_bounds__(kBlock) void k_reduce(
-  const double* __restrict__ partial, int nb, int nv, double* __restrict__ out)
+  const double* __restrict__ partial, int nb, double* __restrict__ out)
 {
   const int v = blockIdx.x;
+  const double* p = partial + (int64_t)v * nb;
   double s = 0.0;
-  for (int b = threadIdx.x; b < nb; b += blockDim.x)
-    s += partial[(int64_t)b * nv + v];
+  for (int b = threadIdx.x; b < nb; b += blockDim.x) s += p[b];
   double a[1] = {s};
   __shared__ double tot[1];
   block_reduce_store<1>(a, tot);
@@ -94,42 +128,96 @@ __global__ __launch_bounds__(kBlock) void k_reduce(
 
 // Fused Arnoldi dots.  Block b = rowblock * ntiles + tile (tiles of one row
 // block are adjacent, so the y/z rows they share are re-read from L2).
-// Tile t covers basis vectors Q_k, k in [8t, 8t+8) and k < nq, and writes
-// partial[b][0..7] = Q_k.y, [8..15] = Q_k.z; tile 0 also writes [16] = y.y,
-// [17] = y.z, [18] = z.z.  z may be null (then its dots are zero).
+// Tile t covers basis vectors Q_k, k in [8t, 8t+8) and k < nq; its value v
+// of row block rb is partial[(t kDotVals + v) nrb + rb]: v = 0..7 Q_k.y,
+// 8..15 Q_k.z, and in tile 0 16 = y.y, 17 = y.z, 18 = z.z.  z may be null
+// (then its dots are zero).
+//
+// Bound by HBM (or the Infinity Cache) on large systems and by the block
+// reduction on small ones: with 2048 row blocks at every size and a
+// butterfly per value it took 23 us at least, 70 us on average at 8,640
+// rows (jacobi, 31 vectors) and 64 us at 960 thousand (FP64, 16 vectors).
 template <typename T>
 __global__ __launch_bounds__(kBlock) void k_arnoldi_dots(
   const T* __restrict__ V, int64_t n, int nq, const T* __restrict__ y,
   const T* __restrict__ z, int ntiles, double* __restrict__ partial)
 {
+  static_assert(kTile == 8, "wave_sum16 reduces 2 kTile sums");
+  constexpr int kVec = 16 / (int)sizeof(T);  // rows of one 16-byte load
+  using Vec = T __attribute__((ext_vector_type(16 / sizeof(T)), aligned(sizeof(T))));
   const int tile = blockIdx.x % ntiles;
   const int rb = blockIdx.x / ntiles;
   const int nrb = gridDim.x / ntiles;
   const int k0 = tile * kTile;
   const int kc = min(kTile, nq - k0);
-  double acc[kDotVals];
+  double acc[16], ex[3] = {0.0, 0.0, 0.0};
 #pragma unroll
-  for (int k = 0; k < kDotVals; ++k) acc[k] = 0.0;
-  const int64_t chunk = (n + nrb - 1) / nrb;
-  const int64_t i0 = (int64_t)rb * chunk;
-  const int64_t i1 = min(n, i0 + chunk);
-  for (int64_t i = i0 + threadIdx.x; i < i1; i += blockDim.x) {
-    const double yi = (double)y[i];
-    const double zi = z ? (double)z[i] : 0.0;
+  for (int k = 0; k < 16; ++k) acc[k] = 0.0;
+  const T* __restrict__ Q = V + (int64_t)k0 * n;
+  auto add = [&](double yi, double zi, const double (&q)[kTile]) {
+#pragma unroll
+    for (int k = 0; k < kTile; ++k) {
+      acc[k] += q[k] * yi;
+      acc[kTile + k] += q[k] * zi;
+    }
+    if (tile == 0) {
+      ex[0] += yi * yi;
+      ex[1] += yi * zi;
+      ex[2] += zi * zi;
+    }
+  };
+  // all blocks of a tile sweep the rows together, 16 bytes of every vector
+  // per lane and step (the vectors start at multiples of sizeof(T) only)
+  for (int64_t i = (int64_t)rb * kBlock + threadIdx.x; i < n / kVec;
+       i += (int64_t)nrb * kBlock) {
+    Vec q[kTile], yv, zv;
 #pragma unroll
     for (int k = 0; k < kTile; ++k)
-      if (k < kc) {
-        const double q = (double)V[(int64_t)(k0 + k) * n + i];
-        acc[k] += q * yi;
-        acc[kTile + k] += q * zi;
-      }
-    if (tile == 0) {
-      acc[2 * kTile] += yi * yi;
-      acc[2 * kTile + 1] += yi * zi;
-      acc[2 * kTile + 2] += zi * zi;
+      if (k < kc)
+        q[k] = *reinterpret_cast<const Vec*>(Q + (int64_t)k * n + kVec * i);
+      else
+        q[k] = (T)0;
+    yv = *reinterpret_cast<const Vec*>(y + kVec * i);
+    if (z)
+      zv = *reinterpret_cast<const Vec*>(z + kVec * i);
+    else
+      zv = (T)0;
+#pragma unroll
+    for (int u = 0; u < kVec; ++u) {
+      double qu[kTile];
+#pragma unroll
+      for (int k = 0; k < kTile; ++k) qu[k] = (double)q[k][u];
+      add((double)yv[u], (double)zv[u], qu);
     }
   }
-  block_reduce_store<kDotVals>(acc, partial + (int64_t)blockIdx.x * kDotVals);
+  // the rows past the last whole vector
+  const int64_t it = n / kVec * kVec + threadIdx.x;
+  if (rb == 0 && it < n) {
+    double qu[kTile];
+#pragma unroll
+    for (int k = 0; k < kTile; ++k) qu[k] = k < kc ? (double)Q[(int64_t)k * n + it] : 0.0;
+    add((double)y[it], z ? (double)z[it] : 0.0, qu);
+  }
+  __shared__ double sh[kBlock / kWave][kDotVals];
+  const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+  if (kc > 0) {
+    const double s = wave_sum16(acc);
+    // lane bits 5..2 chose value bits 3..0
+    if ((lane & 3) == 0) sh[wv][lane >> 2] = s;
+  } else if ((lane & 3) == 0) {
+    sh[wv][lane >> 2] = 0.0;
+  }
+#pragma unroll
+  for (int k = 0; k < 3; ++k) {
+    const double s = tile == 0 ? wave_sum(ex[k]) : 0.0;
+    if (lane == 0) sh[wv][16 + k] = s;
+  }
+  __syncthreads();
+  for (int k = threadIdx.x; k < kDotVals; k += kBlock) {
+    double s = 0.0;
+    for (int w = 0; w < kBlock / kWave; ++w) s += sh[w][k];
+    partial[((int64_t)tile * kDotVals + k) * nrb + rb] = s;
+  }
 }
 
 // Fused Arnoldi update: with Q_k = V[k] (k < nq), y = V[nq], z = V[nq+1]:
@@ -571,7 +659,7 @@ struct Solve {
   // reduce nb x nv partials to nv values and copy them to the host
   int reduce(int nb, int nv, double* host)
   {
-    k_reduce<<<nv, kBlock, 0, st>>>(k->partial, nb, nv, k->red);
+    k_reduce<<<nv, kBlock, 0, st>>>(k->partial, nb, k->red);
     NW_LAUNCH_CHECK();
     NW_HIP(hipMemcpyAsync(k->h_pinned, k->red, sizeof(double) * nv,
                           hipMemcpyDeviceToHost, st));
@@ -664,15 +752,13 @@ struct Solve {
   {
     const int64_t n = k->n;
     const int ntiles = std::max(1, (nq + kTile - 1) / kTile);
-    const int nb = kRowBlocks * ntiles;
-    k_arnoldi_dots<T><<<nb, kBlock, 0, st>>>(
+    const int nrb = dot_row_blocks(n, 16 / (int)sizeof(T), ntiles);
+    k_arnoldi_dots<T><<<nrb * ntiles, kBlock, 0, st>>>(
       V, n, nq, V + (int64_t)nq * n, has_z ? V + (int64_t)(nq + 1) * n : nullptr,
       ntiles, k->partial);
     NW_LAUNCH_CHECK();
-    // reduce per (tile, value) over the row blocks: partial layout is
-    // [rowblock][tile][value] = [rowblock][ntiles * kDotVals]
     std::vector<double> r(ntiles * kDotVals);
-    int rc = reduce(kRowBlocks, ntiles * kDotVals, r.data());
+    int rc = reduce(nrb, ntiles * kDotVals, r.data());
     if (rc) return rc;
     for (int q = 0; q < nq; ++q) {
       const int t = q / kTile, kk = q % kTile;
@@ -709,9 +795,10 @@ struct Solve {
   int residual(const double* x, double* rnorm)
   {
     const int n = (int)k->n;
-    // one pass over the rows, at most kPartialCap partials
-    const int nb = (int)std::min<int64_t>(grid_for((int64_t)n * G, kBlock),
-                                          kPartialCap);
+    // a grid of at most 4096 blocks strides over the rows: the partials of
+    // one block per 256 lanes made the reduction after it, by one workgroup,
+    // cost up to 38 us
+    const int nb = (int)std::min<int64_t>(grid_for((int64_t)n * G, kBlock), 4096);
     switch (G) {
     case 1:
       k_residual<1><<<nb, kBlock, 0, st>>>(c->g.row_ptr, c->g.cols, c->g.vals, x, c->g.rhs, k->r, n, k->partial);
@@ -741,11 +828,12 @@ struct Solve {
   // ||v||^2 and v.w of FP64 vectors (w may equal v)
   int dot64(const double* v, const double* w, double* vw)
   {
-    k_arnoldi_dots<double><<<kRowBlocks, kBlock, 0, st>>>(
+    const int nrb = dot_row_blocks(k->n, 2, 1);
+    k_arnoldi_dots<double><<<nrb, kBlock, 0, st>>>(
       v, k->n, 0, v, w, 1, k->partial);
     NW_LAUNCH_CHECK();
     std::vector<double> r(kDotVals);
-    int rc = reduce(kRowBlocks, kDotVals, r.data());
+    int rc = reduce(nrb, kDotVals, r.data());
     *vw = r[2 * kTile + 1];
     return rc;
   }
