@@ -10,6 +10,7 @@
 #include <vector>
 
 #include "nalu_amd.h"
+#include "nw_geom.h"
 
 namespace nw {
 
@@ -174,16 +175,22 @@ struct Krylov;     // solver workspace (nw_krylov.hip)
 struct AmgDevice;  // AMG hierarchy (nw_amg.hip)
 struct Mpnn;       // learned initial guess (nw_mpnn.hip)
 
+// elements by topology, and where each begins in k_elements' grid
+struct ElemGroups {
+  geom::ElemGroup g[4];
+  int first_block[5] = {0, 0, 0, 0, 0};
+};
+
 // Elements of the mesh and the incidence lists of the device geometry
 // (nw_mesh_elements, nw_compute_geometry); all device arrays.
 struct Geom {
-  int64_t nelem = 0, nhex = 0;
-  int32_t* type = nullptr;   // [nelem] 0 Hex8, 1 Tet4, 2 Wed6, 3 Pyr5
-  int32_t* conn = nullptr;   // [nelem][8]
+  int64_t nelem = 0;
+  ElemGroups groups;
+  int32_t* conn = nullptr;   // [nelem][8], grouped by topology
   int32_t* e_ptr = nullptr;  // [nedge + 1]
-  int32_t* e_inc = nullptr;  // 2 (12 el + s) + flip, element order per edge
+  int32_t* e_inc = nullptr;  // 2 (record of scs) + flip, element order per edge
   int32_t* n_ptr = nullptr;  // [nnode + 1]
-  int32_t* n_inc = nullptr;  // 8 el + a, element order per node
+  int32_t* n_inc = nullptr;  // index of scv, element order per node
   // per-element scratch of nw_compute_geometry (sub-control-surface area
   // vectors and sub-control volumes), allocated with the elements so that a
   // call (e.g. after mesh motion) allocates nothing

@@ -31,5 +31,30 @@ int build_incidence(int64_t nelem, const int32_t* type, const int32_t* conn,
                     std::vector<int32_t>& e_ptr, std::vector<int32_t>& e_inc,
                     std::vector<int32_t>& n_ptr, std::vector<int32_t>& n_inc);
 
+// The elements of one topology: `n` of them from position `first` of the
+// grouped order.  Their SCS scratch is a plane of n area vectors per surface
+// (surface s of the i-th: record scs + s n + i of 24 bytes), their SCV
+// scratch a plane of n values per sub-volume (value scv + a n + i), or the
+// one plane that all four sub-volumes of a tetrahedron share.
+struct ElemGroup {
+  int64_t first = 0, n = 0, scs = 0, scv = 0;
+};
+// planes of the SCV scratch
+constexpr int scv_stored(int topo)
+{
+  return topo == 0 ? 8 : topo == 1 ? 1 : topo == 2 ? 6 : 5;
+}
+
+// Counts the elements by topology and lays out their scratch; *nscs and
+// *nscv: records and values in all.
+void layout_elements(int64_t nelem, const int32_t* type, ElemGroup (&grp)[4],
+                     int64_t* nscs, int64_t* nscv);
+// The connectivity grouped by topology, gconn [nelem][8], and the lists of
+// build_incidence turned into scratch indices: e_inc into 2 (SCS record) +
+// flip, n_inc into SCV values; the lists keep their order.
+void group_elements(int64_t nelem, const int32_t* type, const int32_t* conn,
+                    const ElemGroup (&grp)[4], std::vector<int32_t>& gconn,
+                    std::vector<int32_t>& e_inc, std::vector<int32_t>& n_inc);
+
 }  // namespace geom
 }  // namespace nw

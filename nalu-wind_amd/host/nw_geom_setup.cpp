@@ -39,14 +39,20 @@ int build_incidence(int64_t nelem, const int32_t* type, const int32_t* conn,
                     std::vector<int32_t>& n_ptr, std::vector<int32_t>& n_inc)
 {
   if (nelem < 0 || nelem >= (int64_t{1} << 26)) return NW_E_ARG;
+  int bad = 0;
+#pragma omp parallel for schedule(static) reduction(| : bad)
   for (int64_t el = 0; el < nelem; ++el) {
     const int t = type ? type[el] : 0;
-    if (t < 0 || t > 3) return NW_E_ARG;
+    if (t < 0 || t > 3) {
+      bad = 1;
+      continue;
+    }
     for (int a = 0; a < topo_nodes(t); ++a) {
       const int32_t n = conn[8 * el + a];
-      if (n < 0 || n >= nnode) return NW_E_ARG;
+      bad |= n < 0 || n >= nnode;
     }
   }
+  if (bad) return NW_E_ARG;
   // edges by their smaller node: (larger node, edge id), sorted
   std::vector<int64_t> ap(nnode + 1, 0);
   for (int64_t e = 0; e < nedge; ++e)
@@ -65,7 +71,6 @@ int build_incidence(int64_t nelem, const int32_t* type, const int32_t* conn,
     std::sort(adj.begin() + ap[n], adj.begin() + ap[n + 1]);
   // SCS s of element el -> code 2 (12 el + s) + (L is not the edge's node[0])
   std::vector<int32_t> code((size_t)nelem * 12, -1), eid((size_t)nelem * 12, -1);
-  int bad = 0;
 #pragma omp parallel for schedule(static) reduction(| : bad)
   for (int64_t el = 0; el < nelem; ++el) {
     const int t = type ? type[el] : 0;
@@ -111,6 +116,47 @@ int build_incidence(int64_t nelem, const int32_t* type, const int32_t* conn,
     }
   }
   return NW_OK;
+}
+
+void layout_elements(int64_t nelem, const int32_t* type, ElemGroup (&grp)[4],
+                     int64_t* nscs, int64_t* nscv)
+{
+  for (int64_t el = 0; el < nelem; ++el) ++grp[type ? type[el] : 0].n;
+  *nscs = *nscv = 0;
+  for (int t = 0; t < 4; ++t) {
+    if (t > 0) grp[t].first = grp[t - 1].first + grp[t - 1].n;
+    grp[t].scs = *nscs;
+    grp[t].scv = *nscv;
+    *nscs += grp[t].n * topo_scs(t);
+    *nscv += grp[t].n * scv_stored(t);
+  }
+}
+
+void group_elements(int64_t nelem, const int32_t* type, const int32_t* conn,
+                    const ElemGroup (&grp)[4], std::vector<int32_t>& gconn,
+                    std::vector<int32_t>& e_inc, std::vector<int32_t>& n_inc)
+{
+  std::vector<int32_t> row(nelem);  // of the element within its group
+  int32_t next[4] = {0, 0, 0, 0};
+  for (int64_t el = 0; el < nelem; ++el) row[el] = next[type ? type[el] : 0]++;
+  gconn.resize((size_t)nelem * 8);
+#pragma omp parallel for schedule(static)
+  for (int64_t el = 0; el < nelem; ++el) {
+    const int64_t to = grp[type ? type[el] : 0].first + row[el];
+    std::copy(conn + 8 * el, conn + 8 * el + 8, gconn.begin() + 8 * to);
+  }
+#pragma omp parallel for schedule(static)
+  for (int64_t k = 0; k < (int64_t)e_inc.size(); ++k) {
+    const int64_t i = e_inc[k] >> 1, el = i / 12, s = i % 12;
+    const ElemGroup& g = grp[type ? type[el] : 0];
+    e_inc[k] = (int32_t)(2 * (g.scs + s * g.n + row[el]) + (e_inc[k] & 1));
+  }
+#pragma omp parallel for schedule(static)
+  for (int64_t k = 0; k < (int64_t)n_inc.size(); ++k) {
+    const int64_t el = n_inc[k] >> 3, a = n_inc[k] & 7;
+    const int t = type ? type[el] : 0;
+    n_inc[k] = (int32_t)(grp[t].scv + (t == 1 ? 0 : a) * grp[t].n + row[el]);
+  }
 }
 
 }  // namespace geom
