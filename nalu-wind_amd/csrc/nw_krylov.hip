@@ -11,10 +11,12 @@
 // (Swirydowicz, Langou, Ananthan, Yang, Thomas, "Low synchronization
 // Gram-Schmidt and GMRES algorithms", NLAA 2021): per Arnoldi step one
 // fused dot pass over the basis ([Q, y]^T [y, z]) and one fused update pass
-// that both finishes q_j = (y - Q s)/rho and forms the next candidate, with
-// one host synchronisation.  The Hessenberg column of step j-1 is corrected
-// with the reorthogonalisation coefficients, so every column is final one
-// step after it is first formed.
+// that both finishes q_j = (y - Q s)/rho and forms the next candidate.  The
+// Hessenberg column of step j-1 is corrected with the reorthogonalisation
+// coefficients, so every column is final one step after it is first formed.
+// The column, its Givens rotations and the update's coefficients are computed
+// on the device (k_arnoldi_step); the host only learns, from a word in pinned
+// memory, whether the cycle goes on.
 //
 // Every restart cycle begins from the FP64 residual r = b - A x and ends
 // with x += M^-1 Q y in FP64, so a cycle is one iterative-refinement step.
@@ -126,12 +128,185 @@ __global__ __launch_bounds__(kBlock) void k_reduce(
   if (threadIdx.x == 0) out[v] = tot[0];
 }
 
+// Device state of a cycle (doubles): the unrotated Hessenberg matrix H (the
+// Arnoldi relation A M^-1 Q = Q H) and R, the same columns after the Givens
+// rotations, both column by column; the rotations; the rotated right-hand
+// side; the tentative column; the least-squares solution.
+constexpr int kHsH = 0, kHsR = kHsH + kMaxBasis * kMaxBasis;
+constexpr int kHsCs = kHsR + kMaxBasis * kMaxBasis, kHsSn = kHsCs + kMaxBasis;
+constexpr int kHsG = kHsSn + kMaxBasis, kHsPrev = kHsG + kMaxBasis + 2;
+constexpr int kHsY = kHsPrev + kMaxBasis, kHsRho = kHsY + kMaxBasis;
+constexpr int kHsSize = kHsRho + 1;
+// coef[0] tells the update whether to run; a, c, e, b[], d[] follow
+constexpr int kCoefSize = 4 + 2 * kMaxBasis;
+
+// Ends step j of a cycle (one workgroup): sums the nb partials of each dot
+// (partial[b nv + v]), finishes Hessenberg column j - 1 and rotates it,
+// decides whether the cycle goes on, and if it does forms the tentative
+// column j and the coefficients of the update.  The decision goes to *status
+// (pinned host memory) as token << 16 | stop << 8 | (columns done).
+//
+// A chain of latencies, so its loads are issued together and only the
+// rotations and square roots follow each other: about 4 us where the same
+// on the host (copy of the dots, synchronisation, copy of the coefficients)
+// left the device idle for 12 us.
+__global__ __launch_bounds__(kBlock) void k_arnoldi_step(
+  const double* __restrict__ partial, int nb, int nv, int j, int grow, double beta,
+  double stop_abs, double* __restrict__ hs, double* __restrict__ coef,
+  unsigned long long* __restrict__ status, unsigned long long token)
+{
+  static_assert((kMaxBasis / kTile) * kDotVals <= kBlock, "a thread per dot");
+  constexpr int kParts = kBlock / kWave;
+  const int t = threadIdx.x, q = t & (kWave - 1), part = t / kWave;
+  __shared__ double dots[kBlock], sv[kMaxBasis], tv[kMaxBasis], hc[kMaxBasis + 1],
+    Hp[kParts][kMaxBasis], cs[kMaxBasis], sn[kMaxBasis], rc[kMaxBasis], sums[2];
+  __shared__ bool conv;
+  auto tell = [&](int stop, int kdim) {
+    if (t != 0) return;
+    coef[0] = stop ? 0.0 : 1.0;
+    __hip_atomic_store(status, token << 16 | (unsigned long long)(stop << 8 | kdim),
+                       __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+  };
+  const double prev = t < j ? hs[kHsPrev + t] : 0.0;
+  const double rho_prev = j >= 1 ? hs[kHsRho] : 1.0;
+  const double g_prev = j >= 2 ? hs[kHsG + j - 1] : beta;
+  if (t < j) {
+    cs[t] = hs[kHsCs + t];
+    sn[t] = hs[kHsSn + t];
+  }
+  // the finished columns this thread multiplies by s: l = part mod kParts
+  double hq[kMaxBasis / kParts];
+#pragma unroll
+  for (int u = 0; u < kMaxBasis / kParts; ++u) {
+    const int l = part + u * kParts;
+    hq[u] = l < j - 1 && q <= l + 1 ? hs[kHsH + l * kMaxBasis + q] : 0.0;
+  }
+  double d = 0.0;
+  if (t < nv) {
+#pragma unroll 8
+    for (int b = 0; b < nb; ++b) d += partial[(int64_t)b * nv + t];
+  }
+  dots[t] = d;
+  __syncthreads();
+  const double yy = dots[2 * kTile], yz = dots[2 * kTile + 1];
+  if (!(yy > 0) || !isfinite(yy)) {  // the column j - 1 stays unfinished
+    tell(1, max(j - 1, 0));
+    return;
+  }
+  const double sigma = 1.0 / sqrt(yy);
+  if (t < kMaxBasis) {
+    double a = 0.0, b = 0.0;
+    if (t < j) {
+      const int v = (t / kTile) * kDotVals + t % kTile;
+      a = sigma * dots[v];          // s = Q^T u, u = sigma y
+      b = sigma * dots[v + kTile];  // t = Q^T z
+    }
+    sv[t] = a;
+    tv[t] = b;
+    const double ss = wave_sum(a * a), st = wave_sum(a * b);
+    if (t == 0) {
+      sums[0] = ss;
+      sums[1] = st;
+    }
+  }
+  __syncthreads();
+  const double ss = sums[0], st = sums[1];
+  const double rho = ss < 1.0 ? sqrt(1.0 - ss) : 0.0;
+  if (j >= 1) {
+    // finish column j-1: A M^-1 q_{j-1} = Q (hprev + nu s) + nu rho q_j
+    const double nu = (1.0 / sigma) / rho_prev;
+    if (t <= j) {
+      const double h = t < j ? prev + nu * sv[t] : nu * rho;
+      hs[kHsH + (j - 1) * kMaxBasis + t] = h;
+      hc[t] = h;
+    }
+  }
+  __syncthreads();
+  if (j >= 1 && t == 0) {
+    const int col = j - 1;
+    double a = hc[0];
+#pragma unroll 8
+    for (int k = 0; k < col; ++k) {
+      const double b = hc[k + 1];
+      rc[k] = cs[k] * a + sn[k] * b;
+      a = -sn[k] * a + cs[k] * b;
+    }
+    const double b = hc[j];
+    const double rr = sqrt(a * a + b * b);
+    const double c = rr > 0 ? a / rr : 1.0, s = rr > 0 ? b / rr : 0.0;
+    rc[col] = rr;
+    hs[kHsCs + col] = c;
+    hs[kHsSn + col] = s;
+    hs[kHsG + j] = -s * g_prev;
+    hs[kHsG + col] = c * g_prev;
+    conv = fabs(s * g_prev) <= stop_abs;
+  }
+  // Hs = H[0..j][0..j-1] s, a quarter of the columns per wave
+  {
+    double a = 0.0;
+#pragma unroll
+    for (int u = 0; u < kMaxBasis / kParts; ++u) {
+      const int l = part + u * kParts;
+      if (l < j - 1) a += hq[u] * sv[l];
+    }
+    if (j >= 1 && part == (j - 1) % kParts && q <= j) a += hc[q] * sv[j - 1];
+    Hp[part][q] = a;
+  }
+  __syncthreads();
+  if (t < j) hs[kHsR + (j - 1) * kMaxBasis + t] = rc[t];
+  // converged, end of the cycle or lucky breakdown
+  if ((j >= 1 && conv) || !grow || !(rho > 1e-12)) {
+    tell(1, j);
+    return;
+  }
+  tell(0, j);
+  // tentative column j from the dots of z = A M^-1 u, z = sigma z'
+  //   V[j]   <- q_j = (sigma/rho) y - sum (s_q/rho) Q_q
+  //   V[j+1] <- sigma z' - e sigma y - sum (c_q - e s_q) Q_q
+  auto Hs = [&](int k) { return (Hp[0][k] + Hp[1][k]) + (Hp[2][k] + Hp[3][k]); };
+  static_assert(kParts == 4, "four partial products");
+  const double uz = sigma * sigma * yz, Hj = Hs(j);
+  const double hjj = ((uz - st) / rho - Hj) / rho;
+  const double e = (Hj + rho * hjj) / rho;
+  if (t < j) {
+    const double Ht = Hs(t), h = (tv[t] - Ht) / rho;
+    hs[kHsPrev + t] = h;
+    coef[4 + t] = sv[t] / rho;
+    coef[4 + j + t] = (Ht + rho * h) - e * sv[t];
+  }
+  if (t == 0) {
+    hs[kHsPrev + j] = hjj;
+    hs[kHsRho] = rho;
+    coef[1] = sigma / rho;
+    coef[2] = sigma;
+    coef[3] = e * sigma;
+  }
+}
+
+// The least-squares solution R y = g of a cycle of kdim columns: R staged in
+// LDS, then one wave, lane i holding g_i.
+__global__ __launch_bounds__(kBlock) void k_arnoldi_solve(double* __restrict__ hs, int kdim)
+{
+  __shared__ double R[kMaxBasis * kMaxBasis];
+  for (int i = threadIdx.x; i < kdim * kMaxBasis; i += kBlock)
+    R[i] = (i & (kMaxBasis - 1)) <= i / kMaxBasis ? hs[kHsR + i] : 0.0;
+  const int t = threadIdx.x;
+  double g = t < kdim ? hs[kHsG + t] : 0.0;
+  __syncthreads();
+  if (t >= kWave) return;
+  for (int i = kdim - 1; i >= 0; --i) {
+    const double y = __shfl(g, i) / R[i * kMaxBasis + i];
+    if (t < i) g -= R[i * kMaxBasis + t] * y;
+    if (t == i) hs[kHsY + i] = y;
+  }
+}
+
 // Fused Arnoldi dots.  Block b = rowblock * ntiles + tile (tiles of one row
 // block are adjacent, so the y/z rows they share are re-read from L2).
 // Tile t covers basis vectors Q_k, k in [8t, 8t+8) and k < nq; its value v
-// of row block rb is partial[(t kDotVals + v) nrb + rb]: v = 0..7 Q_k.y,
-// 8..15 Q_k.z, and in tile 0 16 = y.y, 17 = y.z, 18 = z.z.  z may be null
-// (then its dots are zero).
+// of row block rb is value V = t kDotVals + v of partial[V sv + rb sb]: v =
+// 0..7 Q_k.y, 8..15 Q_k.z, and in tile 0 16 = y.y, 17 = y.z, 18 = z.z.  z may
+// be null (then its dots are zero).
 //
 // Bound by HBM (or the Infinity Cache) on large systems and by the block
 // reduction on small ones: with 2048 row blocks at every size and a
@@ -140,7 +315,7 @@ __global__ __launch_bounds__(kBlock) void k_reduce(
 template <typename T>
 __global__ __launch_bounds__(kBlock) void k_arnoldi_dots(
   const T* __restrict__ V, int64_t n, int nq, const T* __restrict__ y,
-  const T* __restrict__ z, int ntiles, double* __restrict__ partial)
+  const T* __restrict__ z, int ntiles, double* __restrict__ partial, int sv, int sb)
 {
   static_assert(kTile == 8, "wave_sum16 reduces 2 kTile sums");
   constexpr int kVec = 16 / (int)sizeof(T);  // rows of one 16-byte load
@@ -216,34 +391,34 @@ __global__ __launch_bounds__(kBlock) void k_arnoldi_dots(
   for (int k = threadIdx.x; k < kDotVals; k += kBlock) {
     double s = 0.0;
     for (int w = 0; w < kBlock / kWave; ++w) s += sh[w][k];
-    partial[((int64_t)tile * kDotVals + k) * nrb + rb] = s;
+    partial[(int64_t)(tile * kDotVals + k) * sv + (int64_t)rb * sb] = s;
   }
 }
 
 // Fused Arnoldi update: with Q_k = V[k] (k < nq), y = V[nq], z = V[nq+1]:
 //   V[nq]   = a y - sum_k b_k Q_k          (the finished basis vector)
 //   V[nq+1] = c z - e y - sum_k d_k Q_k    (the next candidate)
-// coef = {a, c, e, b_0..b_{nq-1}, d_0..d_{nq-1}}.  With has_z == 0 only the
-// first line is applied.
+// coef = {go, a, c, e, b_0..b_{nq-1}, d_0..d_{nq-1}}; go == 0: the cycle has
+// ended and nothing is done.
 template <typename T>
 __global__ __launch_bounds__(kBlock) void k_arnoldi_update(
-  T* __restrict__ V, int64_t n, int nq, const double* __restrict__ coef,
-  int has_z)
+  T* __restrict__ V, int64_t n, int nq, const double* __restrict__ coef)
 {
+  if (coef[0] == 0.0) return;
   __shared__ double cb[kMaxBasis], cd[kMaxBasis];
   for (int k = threadIdx.x; k < nq; k += blockDim.x) {
-    cb[k] = coef[3 + k];
-    cd[k] = coef[3 + nq + k];
+    cb[k] = coef[4 + k];
+    cd[k] = coef[4 + nq + k];
   }
   __syncthreads();
-  const double a = coef[0], c = coef[1], e = coef[2];
+  const double a = coef[1], c = coef[2], e = coef[3];
   T* __restrict__ Y = V + (int64_t)nq * n;
   T* __restrict__ Z = Y + n;
   for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n;
        i += (int64_t)gridDim.x * blockDim.x) {
     const double yi = (double)Y[i];
     double q = a * yi;
-    double w = has_z ? c * (double)Z[i] - e * yi : 0.0;
+    double w = c * (double)Z[i] - e * yi;
     int k = 0;
     for (; k + 4 <= nq; k += 4) {
       const double v0 = (double)V[(int64_t)(k + 0) * n + i];
@@ -259,7 +434,7 @@ __global__ __launch_bounds__(kBlock) void k_arnoldi_update(
       w -= cd[k] * v0;
     }
     Y[i] = (T)q;
-    if (has_z) Z[i] = (T)w;
+    Z[i] = (T)w;
   }
 }
 
@@ -587,6 +762,11 @@ struct Krylov {
   double* partial = nullptr;
   double* red = nullptr;   // reduced results (device)
   double* coef = nullptr;  // coefficients (device)
+  double* hs = nullptr;    // a cycle's small dense state (device)
+  // the steps' decisions in pinned memory, step by step in turn, and the
+  // number of the last step enqueued
+  volatile unsigned long long* status = nullptr;
+  unsigned long long token = 0;
   double* pe = nullptr;    // power iteration work
   double* xg = nullptr;    // learned guess
   int* bad = nullptr;
@@ -620,6 +800,8 @@ void free_krylov(Krylov* k)
   (void)hipFree(k->partial);
   (void)hipFree(k->red);
   (void)hipFree(k->coef);
+  (void)hipFree(k->hs);
+  (void)hipHostFree((void*)k->status);
   (void)hipFree(k->pe);
   (void)hipFree(k->xg);
   (void)hipFree(k->bad);
@@ -744,39 +926,61 @@ struct Solve {
     return spmv<T>(s.mat, v, W, (T)1);
   }
 
-  // Q = V[0..nq), y = V[nq], z = V[nq+1] (if has_z):
-  // qy[k] = Q_k.y, qz[k] = Q_k.z, yy, yz
+  // Enqueues the dots of step j (Q = V[0..j), y = V[j], z = V[j+1] if grow)
+  // and the work that ends the step; its decision arrives under *token.
   template <typename T>
-  int arnoldi_dots(const T* V, int nq, bool has_z, double* qy, double* qz,
-                   double* yy, double* yz)
+  int arnoldi_step(const T* V, int j, bool grow, double beta, double stop_abs,
+                   unsigned long long* token)
   {
     const int64_t n = k->n;
-    const int ntiles = std::max(1, (nq + kTile - 1) / kTile);
+    const int ntiles = std::max(1, (j + kTile - 1) / kTile);
     const int nrb = dot_row_blocks(n, 16 / (int)sizeof(T), ntiles);
+    const int nv = ntiles * kDotVals;
+    // up to kDirect row blocks the step adds their partials itself (a thread
+    // per value, rows of values); more go through a reduction of their own
+    constexpr int kDirect = 48;
+    const bool direct = nrb <= kDirect;
     k_arnoldi_dots<T><<<nrb * ntiles, kBlock, 0, st>>>(
-      V, n, nq, V + (int64_t)nq * n, has_z ? V + (int64_t)(nq + 1) * n : nullptr,
-      ntiles, k->partial);
+      V, n, j, V + (int64_t)j * n, grow ? V + (int64_t)(j + 1) * n : nullptr,
+      ntiles, k->partial, direct ? 1 : nrb, direct ? nv : 1);
+    if (!direct) k_reduce<<<nv, kBlock, 0, st>>>(k->partial, nrb, k->red);
     NW_LAUNCH_CHECK();
-    std::vector<double> r(ntiles * kDotVals);
-    int rc = reduce(nrb, ntiles * kDotVals, r.data());
-    if (rc) return rc;
-    for (int q = 0; q < nq; ++q) {
-      const int t = q / kTile, kk = q % kTile;
-      qy[q] = r[t * kDotVals + kk];
-      qz[q] = r[t * kDotVals + kTile + kk];
-    }
-    *yy = r[2 * kTile];
-    *yz = r[2 * kTile + 1];
+    *token = ++k->token;
+    k_arnoldi_step<<<1, kBlock, 0, st>>>(
+      direct ? k->partial : k->red, direct ? nrb : 1, nv, j, grow ? 1 : 0, beta, stop_abs,
+      k->hs, k->coef, const_cast<unsigned long long*>(k->status) + (*token & 1), *token);
+    NW_LAUNCH_CHECK();
     return NW_OK;
   }
 
-  template <typename T>
-  int arnoldi_update(T* V, int nq, const std::vector<double>& coef, bool has_z)
+  // Waits for the decision of step `token`; the word is written by a kernel
+  // already enqueued, so the wait ends with it or with the stream's error.
+  int step_status(unsigned long long token, bool* stop, int* kdim)
   {
-    NW_HIP(hipMemcpyAsync(k->coef, coef.data(), sizeof(double) * coef.size(),
-                          hipMemcpyHostToDevice, st));
-    k_arnoldi_update<T><<<stream_grid(k->n), kBlock, 0, st>>>(
-      V, k->n, nq, k->coef, has_z ? 1 : 0);
+    const volatile unsigned long long* w = k->status + (token & 1);
+    for (unsigned spin = 1;; ++spin) {
+      const unsigned long long v = *w;
+      if (v >> 16 == token) {
+        *stop = (v >> 8 & 1) != 0;
+        *kdim = (int)(v & 0xff);
+        return NW_OK;
+      }
+      if (spin % 4096 == 0) {
+        const hipError_t e = hipStreamQuery(st);
+        if (e == hipErrorNotReady) {
+          (void)hipGetLastError();  // not an error of a later launch
+          continue;
+        }
+        NW_HIP(e);
+        NW_REQUIRE(*w >> 16 == token, NW_E_HIP, "the solver step left no decision");
+      }
+    }
+  }
+
+  template <typename T>
+  int arnoldi_update(T* V, int nq)
+  {
+    k_arnoldi_update<T><<<stream_grid(k->n), kBlock, 0, st>>>(V, k->n, nq, k->coef);
     NW_LAUNCH_CHECK();
     return NW_OK;
   }
@@ -784,9 +988,7 @@ struct Solve {
   template <typename T>
   int combine(const T* V, int nk, const double* coef, T* u)
   {
-    NW_HIP(hipMemcpyAsync(k->coef, coef, sizeof(double) * nk,
-                          hipMemcpyHostToDevice, st));
-    k_combine<T><<<stream_grid(k->n), kBlock, 0, st>>>(V, k->n, nk, k->coef, u);
+    k_combine<T><<<stream_grid(k->n), kBlock, 0, st>>>(V, k->n, nk, coef, u);
     NW_LAUNCH_CHECK();
     return NW_OK;
   }
@@ -830,7 +1032,7 @@ struct Solve {
   {
     const int nrb = dot_row_blocks(k->n, 2, 1);
     k_arnoldi_dots<double><<<nrb, kBlock, 0, st>>>(
-      v, k->n, 0, v, w, 1, k->partial);
+      v, k->n, 0, v, w, 1, k->partial, nrb, 1);
     NW_LAUNCH_CHECK();
     std::vector<double> r(kDotVals);
     int rc = reduce(nrb, kDotVals, r.data());
@@ -846,102 +1048,41 @@ struct Solve {
   {
     const int64_t n = k->n;
     const int m = std::min(cfg->kspace, max_it);
-    // Hr: unrotated Hessenberg (the Arnoldi relation A M^-1 Q = Q H);
-    // R: the same columns after the Givens rotations (least squares)
-    std::vector<double> Hr((size_t)(m + 1) * m, 0.0), R((size_t)(m + 1) * m, 0.0);
-    std::vector<double> cs(m, 1.0), sn(m, 0.0), g(m + 2, 0.0), sv(kMaxBasis),
-      tv(kMaxBasis), hprev(kMaxBasis, 0.0), Hs(kMaxBasis), hj(kMaxBasis),
-      cv(kMaxBasis), yls(kMaxBasis), coef;
-    auto H = [&](int i, int j) -> double& { return Hr[(size_t)i * m + j]; };
-    auto Rm = [&](int i, int j) -> double& { return R[(size_t)i * m + j]; };
+    // With a cheap operator the steps run one ahead of their decisions: the
+    // host enqueues step j + 1 before it knows whether step j ends the
+    // cycle, so short kernels follow each other without a gap (a step past
+    // the end changes nothing that is read: its column, rotation and basis
+    // vectors lie behind the first kdim).  Under a polynomial or AMG a wasted
+    // application would cost more than the gap, which the update hides.
+    const bool ahead = cfg->precond == NW_PREC_NONE || cfg->precond == NW_PREC_JACOBI;
     T* V = s.V;
     k_convert<T><<<grid_for(n, kBlock), kBlock, 0, st>>>(k->r, V, 1.0 / beta, n);
     NW_LAUNCH_CHECK();
-    g[0] = beta;
-    double rho_prev = 1.0;
-    int kdim = 0;
-    for (int j = 0; j <= m; ++j) {
+    int kdim = 0, rc = NW_OK;
+    bool stop = false;
+    unsigned long long token = 0;
+    for (int j = 0; j <= m && !stop; ++j) {
       const bool grow = j < m;
-      int rc;
       if (grow) {
         rc = apply_op<T>(s, V + (int64_t)j * n, V + (int64_t)(j + 1) * n);
         if (rc) return rc;
       }
-      double yy = 0, yz = 0;
-      rc = arnoldi_dots<T>(V, j, grow, sv.data(), tv.data(), &yy, &yz);
+      const unsigned long long before = token;
+      rc = arnoldi_step<T>(V, j, grow, beta, stop_abs, &token);
+      if (!rc && grow) rc = arnoldi_update<T>(V, j);
+      if (!rc && (!ahead || j > 0)) rc = step_status(ahead ? before : token, &stop, &kdim);
       if (rc) return rc;
-      if (!(yy > 0) || !std::isfinite(yy)) break;
-      const double sigma = 1.0 / std::sqrt(yy);
-      double ss = 0.0;
-      for (int q = 0; q < j; ++q) {
-        sv[q] *= sigma;  // s = Q^T u, u = sigma y
-        ss += sv[q] * sv[q];
-      }
-      const double rho = ss < 1.0 ? std::sqrt(1.0 - ss) : 0.0;
-      if (j >= 1) {
-        // finish column j-1: A M^-1 q_{j-1} = Q (hprev + nu s) + nu rho q_j
-        const int col = j - 1;
-        const double nu = (1.0 / sigma) / rho_prev;
-        for (int q = 0; q < j; ++q) H(q, col) = hprev[q] + nu * sv[q];
-        H(j, col) = nu * rho;
-        for (int q = 0; q <= j; ++q) Rm(q, col) = H(q, col);
-        for (int q = 0; q < col; ++q) {
-          const double a = Rm(q, col), b = Rm(q + 1, col);
-          Rm(q, col) = cs[q] * a + sn[q] * b;
-          Rm(q + 1, col) = -sn[q] * a + cs[q] * b;
-        }
-        const double a = Rm(col, col), b = Rm(col + 1, col);
-        const double rr = std::sqrt(a * a + b * b);
-        cs[col] = rr > 0 ? a / rr : 1.0;
-        sn[col] = rr > 0 ? b / rr : 0.0;
-        Rm(col, col) = rr;
-        Rm(col + 1, col) = 0.0;
-        g[col + 1] = -sn[col] * g[col];
-        g[col] = cs[col] * g[col];
-        ++iters;
-        kdim = j;
-        if (std::fabs(g[col + 1]) <= stop_abs) break;
-      }
-      if (!grow || !(rho > 1e-12)) break;  // end of cycle / lucky breakdown
-      // tentative column j from the dots of z = A M^-1 u, z = sigma z'
-      double st_ = 0.0;
-      for (int q = 0; q < j; ++q) {
-        tv[q] *= sigma;  // t = Q^T z
-        st_ += sv[q] * tv[q];
-      }
-      const double uz = sigma * sigma * yz;
-      for (int q = 0; q <= j; ++q) {  // Hs = H[0..j][0..j-1] s
-        double a = 0.0;
-        for (int l = std::max(0, q - 1); l < j; ++l) a += H(q, l) * sv[l];
-        Hs[q] = a;
-      }
-      for (int q = 0; q < j; ++q) hj[q] = (tv[q] - Hs[q]) / rho;
-      hj[j] = ((uz - st_) / rho - Hs[j]) / rho;
-      for (int q = 0; q <= j; ++q) cv[q] = Hs[q] + rho * hj[q];
-      const double e = cv[j] / rho;
-      // V[j] <- q_j = (sigma/rho) y - sum (s_q/rho) Q_q
-      // V[j+1] <- sigma z' - e sigma y - sum (c_q - e s_q) Q_q
-      coef.assign(3 + 2 * j, 0.0);
-      coef[0] = sigma / rho;
-      coef[1] = sigma;
-      coef[2] = e * sigma;
-      for (int q = 0; q < j; ++q) {
-        coef[3 + q] = sv[q] / rho;
-        coef[3 + j + q] = cv[q] - e * sv[q];
-      }
-      rc = arnoldi_update<T>(V, j, coef, true);
-      if (rc) return rc;
-      for (int q = 0; q <= j; ++q) hprev[q] = hj[q];
-      rho_prev = rho;
     }
+    if (!stop) {
+      rc = step_status(token, &stop, &kdim);
+      if (rc) return rc;
+    }
+    iters += kdim;
     if (kdim == 0) return NW_OK;
     // least squares R y = g, u = Q y, x += M^-1 u
-    for (int i = kdim - 1; i >= 0; --i) {
-      double t = g[i];
-      for (int l = i + 1; l < kdim; ++l) t -= Rm(i, l) * yls[l];
-      yls[i] = t / Rm(i, i);
-    }
-    int rc = combine<T>(V, kdim, yls.data(), s.u);
+    k_arnoldi_solve<<<1, kBlock, 0, st>>>(k->hs, kdim);
+    NW_LAUNCH_CHECK();
+    rc = combine<T>(V, kdim, k->hs + kHsY, s.u);
     if (rc) return rc;
     const T* u = s.u;
     if (cfg->precond == NW_PREC_CHEBYSHEV) {
@@ -1057,7 +1198,12 @@ int nw_linsys_solve(nw_ctx* c, const nw_solver_cfg* cfg, nw_solve_stats* out)
     NW_HIP(hipMalloc(&k->r, sizeof(double) * n));
     NW_HIP(hipMalloc(&k->partial, sizeof(double) * kPartialCap));
     NW_HIP(hipMalloc(&k->red, sizeof(double) * kRedCap));
-    NW_HIP(hipMalloc(&k->coef, sizeof(double) * (3 + 2 * kMaxBasis)));
+    NW_HIP(hipMalloc(&k->coef, sizeof(double) * kCoefSize));
+    NW_HIP(hipMalloc(&k->hs, sizeof(double) * kHsSize));
+    void* hst = nullptr;
+    NW_HIP(hipHostMalloc(&hst, 2 * sizeof(unsigned long long), hipHostMallocCoherent));
+    std::memset(hst, 0, 2 * sizeof(unsigned long long));
+    k->status = static_cast<volatile unsigned long long*>(hst);
     NW_HIP(hipMalloc(&k->bad, sizeof(int)));
     NW_HIP(hipHostMalloc(&k->h_pinned, sizeof(double) * kRedCap));
     NW_HIP(hipEventCreate(&k->ev0));
