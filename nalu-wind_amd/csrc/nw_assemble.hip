@@ -76,10 +76,27 @@ __device__ inline double van_leer(double dqm, double dqp, double eps)
 
 // ------------------------------------------------------------------ physics
 // Each physics type has a Node record of the fields one node contributes,
-// load(n, rec), and edge(e, side, L, R, off, acc) which computes, for the
-// row n = node[side] of edge e:
-//   off[NB]  the (n, other) block of the edge LHS, row-major ndof x ndof
-//   acc[NV]  the (n, n) block contribution (NB values) then rhs(n) (NDOF)
+// load(n, rec), derive(rec) (quantities of the node alone, formed once per
+// record: the row's own node's once per row), and edge(er, me, ot, off, acc)
+// which computes, for the row of `me`, seen from it along the edge to `ot`:
+//   off[NB]  the (me, ot) block of the edge LHS, row-major ndof x ndof
+//   acc[NV]  the (me, me) block contribution (NB values) then rhs(me) (NDOF)
+// The reference's formulas for an edge (L, R) hold for either end with the
+// area vector and the mass flow rate taken out of that end: swapping the ends
+// changes the sign of A, dx, mdot and the fluxes and exchanges the rows.
+// orient(er, side) turns the edge's values out of node[side], so one body
+// serves both ends and the lanes of a wave need not agree on the side.
+//
+// FP64 divisions (about fifteen instructions each) are kept to those that the
+// formulas need per edge: uniform divisors (relaxation, time scale) come as
+// reciprocals from the host, those of a node are in derive().  Momentum had
+// ten per edge end and has one, continuity twelve and has two.  Measured with
+// the common body: momentum 128^3 0.60 -> 0.535 ms (its registers now hold
+// one slot in flight per lane without spilling; two spill and take 0.745),
+// one pass with the Peclet factor 61 x 127 x 45 103 -> 85 us, continuity
+// 192^3 0.730 -> 0.705 ms, mixed 96^3 220 -> 212 us: continuity is bound by
+// its L1 misses (58 M lines of 128 bytes a launch at 192^3, 66 in flight per
+// CU at any time), not by arithmetic, occupancy or loads in flight.
 
 // s, m: buoyancy_source and its mask, loaded only with the balanced
 // buoyancy force (unused registers are dropped otherwise)
@@ -106,7 +123,7 @@ struct ContinuityPhysT {
   using Node = ContNode;
   const double *coords, *vel, *dpdx, *rho, *p, *udiag, *areav;
   int64_t N, E;
-  double nocFac, tauScale, interpTogether, incompressible;
+  double nocFac, invTau, interpTogether, incompressible;
   const double *src, *mask;
   double grav[3];
 
@@ -126,6 +143,16 @@ struct ContinuityPhysT {
     }
   }
 
+  // ud becomes 1 / Udiag, g and s the terms they divide
+  __device__ void derive(Node& r) const
+  {
+    r.ud = 1.0 / r.ud;
+    for (int d = 0; d < 3; ++d) {
+      r.g[d] *= r.ud;
+      if constexpr (BUOY) r.s[d] = (r.m * r.s[d]) * r.ud;
+    }
+  }
+
   struct Edge {
     double av[3];
   };
@@ -135,15 +162,24 @@ struct ContinuityPhysT {
     for (int d = 0; d < 3; ++d) r.av[d] = areav[3 * (int64_t)e + d];
   }
 
-  __device__ void edge(const Edge& er, int side, const Node& L, const Node& R,
+  __device__ void orient(Edge& r, int side) const
+  {
+    for (int d = 0; d < 3; ++d) r.av[d] = side ? -r.av[d] : r.av[d];
+  }
+
+  __device__ void edge(const Edge& er, int, const Node& L, const Node& R,
                        double* off, double* acc) const
   {
     const double om_interpTogether = 1.0 - interpTogether;
     const double om_incomp = 1.0 - incompressible;
     const double* av = er.av;
-    const double projTimeScale = 0.5 * (1.0 / L.ud + 1.0 / R.ud);
+    const double projTimeScale = 0.5 * (L.ud + R.ud);
     const double rhoIp = 0.5 * (L.rho + R.rho);
-    const double denScale = (1.0 / rhoIp) * incompressible + om_incomp;
+    // (1 / rhoIp) incompressible + om_incomp; the quotient is needed only in
+    // the incompressible form (0 times it is 0, or NaN for a zero or NaN rhoIp)
+    const double denScale = incompressible != 0.0
+                              ? (1.0 / rhoIp) * incompressible + om_incomp
+                              : (fabs(rhoIp) > 0.0 ? om_incomp : __builtin_nan(""));
     double dx[3];
     double axdx = 0.0, asq = 0.0;
     for (int d = 0; d < 3; ++d) {
@@ -162,19 +198,18 @@ struct ContinuityPhysT {
       const double kxj = av[d] - asq * inv_axdx * dx[d];
       const double rhoUjIp = 0.5 * (R.rho * R.u[d] + L.rho * L.u[d]);
       const double ujIp = 0.5 * (R.u[d] + L.u[d]);
-      double GjIp = 0.5 * (R.g[d] / R.ud + L.g[d] / L.ud);
-      if constexpr (BUOY)
-        GjIp -= 0.5 * ((R.m * R.s[d]) / R.ud + (L.m * L.s[d]) / L.ud);
+      double GjIp = 0.5 * (R.g[d] + L.g[d]);
+      if constexpr (BUOY) GjIp -= 0.5 * (R.s[d] + L.s[d]);
       tmdot += (interpTogether * rhoUjIp + om_interpTogether * rhoIp * ujIp +
                 GjIp) * av[d] -
                kxj * GjIp * nocFac;
     }
-    tmdot /= tauScale;
+    tmdot *= invTau;
     tmdot *= denScale;
-    const double lhsfac = -asq * inv_axdx * projTimeScale * denScale / tauScale;
+    const double lhsfac = -asq * inv_axdx * projTimeScale * denScale * invTau;
     off[0] = lhsfac;   // lhs(0,1) == lhs(1,0)
     acc[0] = -lhsfac;  // lhs(0,0) == lhs(1,1)
-    acc[1] = side ? tmdot : -tmdot;
+    acc[1] = -tmdot;
   }
 };
 
@@ -190,7 +225,7 @@ struct ScalarPhys {
   using Node = ScalNode;
   const double *coords, *vrtm, *q, *dqdx, *rho, *dflux, *areav, *mdotf;
   int64_t N, E;
-  double alpha, alphaUpw, hoUpwind, relaxFac;
+  double alpha, alphaUpw, hoUpwind, invRelax;
   int useLimiter;
   PecletDev pec;
 
@@ -206,9 +241,18 @@ struct ScalarPhys {
     r.dflux = dflux[n];
   }
 
+  // rho becomes the kinematic coefficient dflux / rho
+  __device__ void derive(Node& r) const { r.rho = r.dflux / r.rho; }
+
   struct Edge {
     double av[3], mdot;
   };
+
+  __device__ void orient(Edge& r, int side) const
+  {
+    for (int d = 0; d < 3; ++d) r.av[d] = side ? -r.av[d] : r.av[d];
+    r.mdot = side ? -r.mdot : r.mdot;
+  }
 
   __device__ void load_edge(int e, Edge& r) const
   {
@@ -216,7 +260,7 @@ struct ScalarPhys {
     r.mdot = mdotf[e];
   }
 
-  __device__ void edge(const Edge& er, int side, const Node& L, const Node& R,
+  __device__ void edge(const Edge& er, int, const Node& L, const Node& R,
                        double* off, double* acc) const
   {
     const double eps = 1.0e-16;
@@ -225,7 +269,7 @@ struct ScalarPhys {
     const double mdot = er.mdot;
     const double qNp1L = L.q, qNp1R = R.q;
     const double viscIp = 0.5 * (L.dflux + R.dflux);
-    const double diffIp = 0.5 * (L.dflux / L.rho + R.dflux / R.rho);
+    const double diffIp = 0.5 * (L.rho + R.rho);
     double dx[3];
     double axdx = 0.0, asq = 0.0, udotx = 0.0;
     for (int d = 0; d < 3; ++d) {
@@ -255,9 +299,6 @@ struct ScalarPhys {
     const double qIpR = qNp1R - dqR * hoUpwind * limitR;
     const double lhsfac = -viscIp * asq * inv_axdx;
     const double diffFlux = lhsfac * (qNp1R - qNp1L) + nonOrth;
-    double l00 = -lhsfac / relaxFac, l01 = lhsfac, l10 = lhsfac,
-           l11 = -lhsfac / relaxFac;
-    double r0 = -diffFlux, r1 = diffFlux;
     const double qIp = 0.5 * (qNp1R + qNp1L);
     const double qUpw = (mdot > 0) ? (alphaUpw * qIpL + om_alphaUpw * qIp)
                                    : (alphaUpw * qIpR + om_alphaUpw * qIp);
@@ -265,24 +306,14 @@ struct ScalarPhys {
     const double qHatR = (alpha * qIpR + om_alpha * qIp);
     const double qCds = 0.5 * (qHatL + qHatR);
     const double adv_flux = mdot * (pecfac * qUpw + om_pecfac * qCds);
-    r0 -= adv_flux;
-    r1 += adv_flux;
-    double alhsfac = 0.5 * (mdot + fabs(mdot)) * pecfac * alphaUpw +
-                     0.5 * alpha * om_pecfac * mdot;
-    l00 += alhsfac / relaxFac;
-    l10 -= alhsfac;
-    alhsfac = 0.5 * (mdot - fabs(mdot)) * pecfac * alphaUpw +
-              0.5 * alpha * om_pecfac * mdot;
-    l11 -= alhsfac / relaxFac;
-    l01 += alhsfac;
-    alhsfac = 0.5 * mdot * (pecfac * om_alphaUpw + om_pecfac * om_alpha);
-    l00 += alhsfac / relaxFac;
-    l01 += alhsfac;
-    l10 -= alhsfac;
-    l11 -= alhsfac / relaxFac;
-    off[0] = side ? l10 : l01;
-    acc[0] = side ? l11 : l00;
-    acc[1] = side ? r1 : r0;
+    const double alhsL = 0.5 * (mdot + fabs(mdot)) * pecfac * alphaUpw +
+                         0.5 * alpha * om_pecfac * mdot;
+    const double alhsR = 0.5 * (mdot - fabs(mdot)) * pecfac * alphaUpw +
+                         0.5 * alpha * om_pecfac * mdot;
+    const double alhsC = 0.5 * mdot * (pecfac * om_alphaUpw + om_pecfac * om_alpha);
+    off[0] = lhsfac + alhsR + alhsC;
+    acc[0] = -lhsfac * invRelax + alhsL * invRelax + alhsC * invRelax;
+    acc[1] = -diffFlux - adv_flux;
   }
 };
 
@@ -295,7 +326,7 @@ struct MomNodeT {
 };
 template <>
 struct MomNodeT<true> {
-  double x[3], u[3], g[9], visc, wall, rho;
+  double x[3], u[3], g[9], visc, wall, nu;
 };
 template <bool PEC>
 struct MomEdgeT {
@@ -310,7 +341,7 @@ struct MomEdgeT<true> {
 template <bool PEC>
 struct MomentumPhysT {
   static constexpr int NDOF = 3;
-  static constexpr int kLanes = 2, kUnroll = 2, kUnroll2 = 2, kMinWaves = 2;
+  static constexpr int kLanes = 2, kUnroll = 1, kUnroll2 = 1, kMinWaves = 2;
   // persistent: 0.577 vs 0.643 ms on the 128^3 box; with the Peclet factor
   // in the kernel (18 dwords of spill, 33 persistent) it is slower (0.95 vs
   // 0.76 ms per step)
@@ -321,7 +352,7 @@ struct MomentumPhysT {
   using Edge = MomEdgeT<PEC>;
   const double *coords, *vel, *dudx, *visc, *areav, *mdotf, *pecfacf, *wall;
   int64_t N, E;
-  double alpha, alphaUpw, hoUpwind, relaxFacU, includeDivU;
+  double alpha, alphaUpw, hoUpwind, invRelaxU, includeDivU;
   int useLimiter;
   // PEC only: density in, the edge Peclet number and factor out (written
   // once, by the L end's row)
@@ -338,7 +369,19 @@ struct MomentumPhysT {
     for (int k = 0; k < 9; ++k) r.g[k] = dudx[9 * (int64_t)n + k];
     r.visc = visc[n];
     r.wall = wall[n];
-    if constexpr (PEC) r.rho = rho[n];
+    if constexpr (PEC) r.nu = rho[n];
+  }
+
+  // with PEC nu, loaded as the density, becomes visc / rho
+  __device__ void derive(Node& r) const
+  {
+    if constexpr (PEC) r.nu = r.visc / r.nu;
+  }
+
+  __device__ void orient(Edge& r, int side) const
+  {
+    for (int d = 0; d < 3; ++d) r.av[d] = side ? -r.av[d] : r.av[d];
+    r.mdot = side ? -r.mdot : r.mdot;
   }
 
   __device__ void load_edge(int e, Edge& r) const
@@ -358,7 +401,7 @@ struct MomentumPhysT {
   {
     if constexpr (PEC) {
       const double eps = 1.0e-16;
-      const double diffIp = 0.5 * (L.visc / L.rho + R.visc / R.rho);
+      const double diffIp = 0.5 * (L.nu + R.nu);
       double udotx = 0.0;
       for (int d = 0; d < 3; ++d) {
         const double dxj = R.x[d] - L.x[d];
@@ -437,7 +480,9 @@ struct MomentumPhysT {
                          0.5 * alpha * om_pecfac * mdot;
     const double alhsC =
       0.5 * mdot * (pecfac * om_alphaUpw + om_pecfac * om_alpha);
-    const double r = relaxFacU;
+    const double ir = invRelaxU;
+    const double dii = alhsL * ir + alhsC * ir - dlhsfac * ir;
+    const double oii = alhsR + alhsC + dlhsfac;
     double divU = 0.0;
     for (int j = 0; j < 3; ++j) divU += duidxj[j][j];
     for (int i = 0; i < 3; ++i) {
@@ -454,32 +499,14 @@ struct MomentumPhysT {
       for (int j = 0; j < 3; ++j)
         diff_flux += -viscIp * (duidxj[i][j] + duidxj[j][i]) * av[j];
       const double total_flux = adv_flux + diff_flux * mask;
-      // this side's rows: (rowL,rowL)/(rowL,rowR) or (rowR,rowR)/(rowR,rowL)
-      double dii, oii;
-      if (side == 0) {
-        dii = alhsL / r;
-        dii += alhsC / r;
-        dii -= dlhsfac / r;
-        oii = alhsR;
-        oii += alhsC;
-        oii += dlhsfac;
-        acc[9 + i] = -total_flux;
-      } else {
-        dii = -(alhsR / r);
-        dii -= alhsC / r;
-        dii -= dlhsfac / r;
-        oii = -alhsL;
-        oii -= alhsC;
-        oii += dlhsfac;
-        acc[9 + i] = total_flux;
-      }
+      acc[9 + i] = -total_flux;
       for (int j = 0; j < 3; ++j) {
         const double lhsfacNS = -viscIp * av[i] * av[j] * inv_axdx;
         if (j == i) {
-          acc[3 * i + j] = dii - lhsfacNS / r;
+          acc[3 * i + j] = dii - lhsfacNS * ir;
           off[3 * i + j] = oii + lhsfacNS;
         } else {
-          acc[3 * i + j] = -(lhsfacNS / r);
+          acc[3 * i + j] = -(lhsfacNS * ir);
           off[3 * i + j] = lhsfacNS;
         }
       }
@@ -540,10 +567,9 @@ __device__ inline void walk_row(const P& phys, const typename P::Node& me,
     for (int u = 0; u < U; ++u) {
       if (!ok[u]) continue;
       double off[NB], con[NV];
-      if (c[u] & 1)
-        phys.edge(er[u], 1, ot[u], me, off, con);
-      else
-        phys.edge(er[u], 0, me, ot[u], off, con);
+      phys.derive(ot[u]);
+      phys.orient(er[u], c[u] & 1);
+      phys.edge(er[u], c[u] & 1, me, ot[u], off, con);
       put(sl[u], off);
       for (int v = 0; v < NV; ++v) acc[v] += con[v];
     }
@@ -668,6 +694,7 @@ __device__ inline void assemble_task(
     r_diag = diag[row];
     if (skip) skipped = skip[row] != 0;
     phys.load(row, me);
+    phys.derive(me);
   }
   double acc[NV];
   for (int v = 0; v < NV; ++v) acc[v] = 0.0;
@@ -1188,14 +1215,14 @@ int nw_assemble_continuity(nw_ctx* c, const nw_continuity_opts* o)
     NW_GET(NW_F_BUOYANCY_SOURCE, src);
     NW_GET(NW_F_BUOYANCY_SOURCE_MASK, mask);
     ContinuityPhysT<true> P{coords, vel, dpdx, rho, p, udiag, areav, c->nnode,
-                            c->nedge, o->noc, o->dt / o->gamma1,
+                            c->nedge, o->noc, 1.0 / (o->dt / o->gamma1),
                             o->interp_together, o->incompressible, src, mask,
                             {o->gravity[0], o->gravity[1], o->gravity[2]}};
     return check_system_finite(c, launch_rows(c, P, o->accumulate),
                                "ContinuityEdgeSolverAlg");
   }
   ContinuityPhysT<false> P{coords, vel, dpdx, rho, p, udiag, areav, c->nnode,
-                           c->nedge, o->noc, o->dt / o->gamma1,
+                           c->nedge, o->noc, 1.0 / (o->dt / o->gamma1),
                            o->interp_together, o->incompressible, nullptr,
                            nullptr, {0.0, 0.0, 0.0}};
   return check_system_finite(c, launch_rows(c, P, o->accumulate),
@@ -1215,7 +1242,7 @@ int nw_assemble_scalar(nw_ctx* c, const nw_scalar_opts* o)
   NW_GET(NW_E_AREA_VECTOR, areav);
   NW_GET(NW_E_MASS_FLOW_RATE, mdot);
   ScalarPhys P{coords, vel, q, dqdx, rho, dflux, areav, mdot, c->nnode, c->nedge,
-               o->alpha, o->alpha_upw, o->upw, o->relax, o->use_limiter,
+               o->alpha, o->alpha_upw, o->upw, 1.0 / o->relax, o->use_limiter,
                PecletDev{o->peclet.form, o->peclet.hybrid, o->peclet.c1,
                          o->peclet.c2}};
   return check_system_finite(c, launch_rows(c, P, o->accumulate),
@@ -1236,7 +1263,7 @@ int nw_assemble_momentum(nw_ctx* c, const nw_momentum_opts* o)
   NW_GET(NW_E_PECLET_FACTOR, pecfac);
   MomentumPhysT<false> P{coords, vel, dudx, visc, areav, mdot, pecfac, wall,
                          c->nnode, c->nedge, o->alpha, o->alpha_upw, o->upw,
-                         o->relax, o->include_divU, o->use_limiter,
+                         1.0 / o->relax, o->include_divU, o->use_limiter,
                          nullptr, nullptr, nullptr, PecletDev{}};
   double* xdiag = nullptr;
   if (o->extract_diagonal) {
@@ -1267,7 +1294,7 @@ int nw_assemble_momentum_with_peclet(nw_ctx* c, const nw_momentum_opts* o,
   if (rc) return rc;
   MomentumPhysT<true> P{coords, vel, dudx, visc, areav, mdot, nullptr, wall,
                         c->nnode, c->nedge, o->alpha, o->alpha_upw, o->upw,
-                        o->relax, o->include_divU, o->use_limiter,
+                        1.0 / o->relax, o->include_divU, o->use_limiter,
                         rho, pn, pfac,
                         PecletDev{pf->form, pf->hybrid, pf->c1, pf->c2}};
   double* xdiag = nullptr;
