@@ -7,6 +7,18 @@
 // It runs in the solver's storage type: double for the FP64 method, float
 // for the FP32-inner method (the FP32 copy is narrowed from the FP64 one on
 // the device and shares its structure arrays).
+//
+// Every level works on its operator with the columns scaled to a unit
+// diagonal, B = A D^-1, and on the iterate x^ = D x: then A x = B x^, the
+// residual and the restriction are as they were, the smoother's D^-1 is gone
+// (d^ = c1 d^ + c2 (b - B z^)), the prolongators become D P D_c^-1, and the
+// V-cycle returns D M^-1 b, which A M^-1 b = B (D M^-1 b) and the solver's
+// update x += D^-1 x^ take as it is.  Degree 2 from zero is then
+//   x^ = alpha v - beta B v,  alpha = (1 + c1)/theta + c2, beta = c2/theta,
+// one pass that reads the matrix and v and writes x^, where the starting
+// term, d and z were vectors of their own (fine level, FP64: 5 vectors of
+// traffic per smoothing beside the matrix instead of 10 before the coarse
+// correction, 6 instead of 13 after it).
 #include <algorithm>
 #include <chrono>
 #include <cmath>
@@ -20,33 +32,48 @@ namespace nw {
 
 namespace {
 
-__global__ void k_dense_mv(const double* __restrict__ M, int n,
-                           const double* __restrict__ x, double* __restrict__ y)
-{
-  const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= n) return;
-  double s = 0.0;
-  for (int j = 0; j < n; ++j) s += M[(int64_t)i * n + j] * x[j];
-  y[i] = s;
-}
-
-__global__ void k_dense_mv_f(const float* __restrict__ M, int n,
-                             const float* __restrict__ x, float* __restrict__ y)
-{
-  const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= n) return;
-  double s = 0.0;
-  for (int j = 0; j < n; ++j) s += (double)M[(int64_t)i * n + j] * (double)x[j];
-  y[i] = (float)s;
-}
-
+// y = M x, the coarsest level's dense inverse: one wave per row, FP64 sums
+// (a lane per row walked its row alone, each load 64 rows apart: 100 us for
+// 265 rows).
 template <typename T>
-__global__ void k_axpy_t(T* __restrict__ x, const T* __restrict__ t, int n)
+__global__ __launch_bounds__(kBlock) void k_dense_mv(const T* __restrict__ M, int n,
+                                                    const T* __restrict__ x, T* __restrict__ y)
 {
-  const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i < n) x[i] += t[i];
+  const int i = (int)((blockIdx.x * kBlock + threadIdx.x) / kWave);
+  if (i >= n) return;
+  const int lane = threadIdx.x & (kWave - 1);
+  double s = 0.0;
+#pragma unroll 4
+  for (int j = lane; j < n; j += kWave) s += (double)M[(int64_t)i * n + j] * (double)x[j];
+  for (int o = kWave / 2; o > 0; o >>= 1) s += __shfl_xor(s, o);
+  if (lane == 0) y[i] = (T)s;
 }
 
+// Scales a stored matrix by rows and columns in place: v[p] *= row(r) / col(c)
+// factors, rinv and cinv holding the inverses 1 / row and 1 / col of the
+// diagonals (0: an empty row, scaled to 0); either may be null.  A lane per
+// row in sliced ELL form (sp) or CSR (rp).
+__global__ __launch_bounds__(kBlock) void k_scale_mat(
+  const int64_t* __restrict__ sp, const int32_t* __restrict__ rp, const int32_t* __restrict__ ci,
+  double* __restrict__ v, int n, const double* __restrict__ rinv,
+  const double* __restrict__ cinv)
+{
+  const int r = blockIdx.x * blockDim.x + threadIdx.x;
+  if (r >= n) return;
+  double f = 1.0;
+  if (rinv) f = rinv[r] != 0.0 ? 1.0 / rinv[r] : 0.0;
+  int64_t p, end, step;
+  if (sp) {
+    p = sp[r >> 6] + (r & 63);
+    end = sp[(r >> 6) + 1];
+    step = 64;
+  } else {
+    p = rp[r];
+    end = rp[r + 1];
+    step = 1;
+  }
+  for (; p < end; p += step) v[p] *= cinv ? f * cinv[ci[p]] : f;
+}
 
 }  // namespace
 
@@ -63,12 +90,13 @@ struct DevMat {
   const int32_t* ci = nullptr;
   const int32_t* dia_w = nullptr;  // offset and delta forms of the fine
   const int32_t* dia_off = nullptr;  // level's slices
-  const int8_t* d16 = nullptr;
-  const int16_t* cd = nullptr;
-  T* v = nullptr;
+  const int32_t* base = nullptr;
+  const uint16_t* cd = nullptr;
+  const T* v = nullptr;
   int64_t nv = 0;  // stored values (padding included)
-  SellView view() const { return {sp, ci, dia_w, dia_off, d16, cd}; }
-  int64_t* own_sp = nullptr;
+  SellView view() const { return {sp, ci, dia_w, dia_off, base, cd}; }
+  T* own_v = nullptr;  // v, but for the fine level (the solver's copy)
+  Sell own;            // sliced ELL structure
   int32_t* own_rp = nullptr;
   int32_t* own_ci = nullptr;
 };
@@ -111,46 +139,28 @@ static void mat_resid(const DevMat<T>& M, const T* x, const T* b, T* r,
     NW_ROW_LAUNCH(k_resid, T, M.G, M.n, st, M.rp, M.ci, M.v, x, b, r, M.n);
 }
 
-// zo = z + d after the step, or with add zo += z + d
+// out = alpha v - beta A v, with add added to out
 template <typename T>
-static void mat_cheb_step(const DevMat<T>& M, const T* z, const T* v,
-                          const T* dinv, T* d, T* zo, T c1, T c2, bool add,
-                          hipStream_t st)
+static void mat_smooth(const DevMat<T>& M, const T* v, T* out, T alpha, T beta, bool add,
+                       hipStream_t st)
 {
   if (M.sp && add)
-    k_sell_cheb_step<T, true><<<grid_for(M.n, kBlock), kBlock, 0, st>>>(
-      M.view(), M.v, z, v, dinv, d, zo, M.n, c1, c2);
+    k_sell_smooth<T, true><<<grid_for(M.n, kBlock), kBlock, 0, st>>>(M.view(), M.v, v, out,
+                                                                     M.n, alpha, beta);
   else if (M.sp)
-    k_sell_cheb_step<T><<<grid_for(M.n, kBlock), kBlock, 0, st>>>(
-      M.view(), M.v, z, v, dinv, d, zo, M.n, c1, c2);
+    k_sell_smooth<T><<<grid_for(M.n, kBlock), kBlock, 0, st>>>(M.view(), M.v, v, out, M.n,
+                                                               alpha, beta);
   else if (add)
-    NW_ROW_LAUNCH_ADD(k_cheb_step, T, M.G, M.n, st, M.rp, M.ci, M.v, z, v,
-                      dinv, d, zo, M.n, c1, c2);
+    NW_ROW_LAUNCH_ADD(k_smooth, T, M.G, M.n, st, M.rp, M.ci, M.v, v, out, M.n, alpha, beta);
   else
-    NW_ROW_LAUNCH(k_cheb_step, T, M.G, M.n, st, M.rp, M.ci, M.v, z, v, dinv,
-                  d, zo, M.n, c1, c2);
-}
-
-// r = b - A x, then d = z = dinv r inv_theta
-template <typename T>
-static void mat_resid_cheb_init(const DevMat<T>& M, const T* x, const T* b,
-                                T* r, const T* dinv, T* d, T* z, T inv_theta,
-                                hipStream_t st)
-{
-  if (M.sp)
-    k_sell_resid_cheb_init<T><<<grid_for(M.n, kBlock), kBlock, 0, st>>>(
-      M.view(), M.v, x, b, r, dinv, d, z, M.n, inv_theta);
-  else
-    NW_ROW_LAUNCH(k_resid_cheb_init, T, M.G, M.n, st, M.rp, M.ci, M.v, x, b,
-                  r, dinv, d, z, M.n, inv_theta);
+    NW_ROW_LAUNCH(k_smooth, T, M.G, M.n, st, M.rp, M.ci, M.v, v, out, M.n, alpha, beta);
 }
 
 template <typename T>
 struct DevLevel {
   DevMat<T> A, P, R;
-  T* dinv = nullptr;
-  T *x = nullptr, *b = nullptr, *r = nullptr, *t = nullptr;
-  T *cd = nullptr, *cz = nullptr, *cz2 = nullptr;
+  double* dinv = nullptr;  // FP64 hierarchy only
+  T *x = nullptr, *b = nullptr, *r = nullptr;
   double lmax = 0;
   int n = 0;
 };
@@ -169,17 +179,16 @@ struct AmgDevice {
   std::vector<int64_t> rows, nnz;  // per level
   int nlev = 0;
   double setup_seconds = 0;
-  int cheb_degree = 2;
   double cheb_ratio = 20.0;
 };
 
 template <typename T>
 static void free_mat(DevMat<T>& m)
 {
-  (void)hipFree(m.own_sp);
+  sell_free(m.own);
   (void)hipFree(m.own_rp);
   (void)hipFree(m.own_ci);
-  (void)hipFree(m.v);
+  (void)hipFree(m.own_v);
   m = DevMat<T>();
 }
 
@@ -190,7 +199,8 @@ static void free_hier(DevHier<T>& h)
     free_mat(L.A);
     free_mat(L.P);
     free_mat(L.R);
-    for (T* p : {L.dinv, L.x, L.b, L.r, L.t, L.cd, L.cz, L.cz2}) (void)hipFree(p);
+    (void)hipFree(L.dinv);
+    for (T* p : {L.x, L.b, L.r}) (void)hipFree(p);
   }
   h.lv.clear();
   (void)hipFree(h.cinv);
@@ -424,14 +434,15 @@ static int upload_mat(const amg::Csr& h, DevMat<double>& d, hipStream_t st)
     d.nv = nnz;
     NW_HIP(hipMalloc(&d.own_rp, sizeof(int32_t) * rp.size()));
     NW_HIP(hipMalloc(&d.own_ci, sizeof(int32_t) * std::max<int64_t>(nnz, 1)));
-    NW_HIP(hipMalloc(&d.v, sizeof(double) * std::max<int64_t>(nnz, 1)));
+    NW_HIP(hipMalloc(&d.own_v, sizeof(double) * std::max<int64_t>(nnz, 1)));
     d.rp = d.own_rp;
     d.ci = d.own_ci;
+    d.v = d.own_v;
     NW_HIP(hipMemcpyAsync(d.own_rp, rp.data(), sizeof(int32_t) * rp.size(),
                           hipMemcpyHostToDevice, st));
     NW_HIP(hipMemcpyAsync(d.own_ci, h.ci.data(), sizeof(int32_t) * nnz,
                           hipMemcpyHostToDevice, st));
-    NW_HIP(hipMemcpyAsync(d.v, h.v.data(), sizeof(double) * nnz, hipMemcpyHostToDevice, st));
+    NW_HIP(hipMemcpyAsync(d.own_v, h.v.data(), sizeof(double) * nnz, hipMemcpyHostToDevice, st));
     NW_HIP(hipStreamSynchronize(st));
     return NW_OK;
   }
@@ -445,22 +456,24 @@ static int upload_mat(const amg::Csr& h, DevMat<double>& d, hipStream_t st)
   NW_HIP(hipMemcpyAsync(drp, rp.data(), sizeof(int32_t) * (n + 1), hipMemcpyHostToDevice, st));
   NW_HIP(hipMemcpyAsync(dci, h.ci.data(), sizeof(int32_t) * nnz, hipMemcpyHostToDevice, st));
   NW_HIP(hipMemcpyAsync(dv, h.v.data(), sizeof(double) * nnz, hipMemcpyHostToDevice, st));
-  Sell s;
+  Sell& s = d.own;  // owned by d, also after a failure
   rc = sell_build(drp, dci, (int)n, s, st, true);
-  d.own_sp = s.sp;  // owned by d from here on, also on failure
-  d.own_ci = s.ci;
-  tmp.p.push_back(s.slot);
   if (rc) return rc;
   d.sp = s.sp;
   d.ci = s.ci;
+  d.base = s.base;
+  d.cd = s.cd;
   d.nv = s.len;
-  NW_HIP(hipMalloc(&d.v, sizeof(double) * std::max<int64_t>(s.len, 1)));
+  NW_HIP(hipMalloc(&d.own_v, sizeof(double) * std::max<int64_t>(s.len, 1)));
+  d.v = d.own_v;
   if (s.len > 0) {
     k_sell_values<double><<<grid_for(s.len, kBlock), kBlock, 0, st>>>(s.slot, s.ci, dv,
-                                                                      nullptr, d.v, s.len);
+                                                                      nullptr, d.own_v, s.len);
     NW_LAUNCH_CHECK();
   }
   NW_HIP(hipStreamSynchronize(st));
+  (void)hipFree(s.slot);  // the values are in place
+  s.slot = nullptr;
   return NW_OK;
 }
 
@@ -473,10 +486,13 @@ static int narrow_mat(const DevMat<double>& s, DevMat<float>& d, hipStream_t st)
   d.sp = s.sp;
   d.rp = s.rp;
   d.ci = s.ci;
+  d.base = s.base;
+  d.cd = s.cd;
   d.nv = s.nv;
-  NW_HIP(hipMalloc(&d.v, sizeof(float) * std::max<int64_t>(s.nv, 1)));
+  NW_HIP(hipMalloc(&d.own_v, sizeof(float) * std::max<int64_t>(s.nv, 1)));
+  d.v = d.own_v;
   if (s.nv > 0) {
-    k_narrow<float><<<grid_for(s.nv, kBlock), kBlock, 0, st>>>(s.v, d.v, s.nv);
+    k_narrow<float><<<grid_for(s.nv, kBlock), kBlock, 0, st>>>(s.v, d.own_v, s.nv);
     NW_LAUNCH_CHECK();
   }
   return NW_OK;
@@ -485,7 +501,7 @@ static int narrow_mat(const DevMat<double>& s, DevMat<float>& d, hipStream_t st)
 template <typename T>
 static int alloc_level_vectors(DevLevel<T>& L)
 {
-  for (T** p : {&L.x, &L.b, &L.r, &L.t, &L.cd, &L.cz, &L.cz2})
+  for (T** p : {&L.x, &L.b, &L.r})
     NW_HIP(hipMalloc(p, sizeof(T) * std::max(L.n, 1)));
   return NW_OK;
 }
@@ -503,7 +519,7 @@ static int upload_hier(Ctx* c, const amg::Hierarchy& h, DevHier<double>& H)
     L.lmax = hl.lmax;
     if (l == 0) {
       // the fine operator is the linear system's own matrix, in the
-      // graph's sliced ELL order (values refreshed at every solve)
+      // graph's sliced ELL order (the solver's copy, made at every solve)
       NW_REQUIRE(c->g.sell.ci && L.n == c->g.nnode, NW_E_STATE,
                  "sliced ELL form not built");
       L.A.n = L.n;
@@ -511,10 +527,9 @@ static int upload_hier(Ctx* c, const amg::Hierarchy& h, DevHier<double>& H)
       L.A.ci = c->g.sell.ci;
       L.A.dia_w = c->g.sell.dia_w;
       L.A.dia_off = c->g.sell.dia_off;
-      L.A.d16 = c->g.sell.d16;
+      L.A.base = c->g.sell.base;
       L.A.cd = c->g.sell.cd;
       L.A.nv = c->g.sell.len;
-      NW_HIP(hipMalloc(&L.A.v, sizeof(double) * std::max<int64_t>(c->g.sell.len, 1)));
     } else {
       int rc = upload_mat(hl.A, L.A, st);
       if (rc) return rc;
@@ -528,8 +543,14 @@ static int upload_hier(Ctx* c, const amg::Hierarchy& h, DevHier<double>& H)
     if (rc) return rc;
   }
   H.nc = (int)h.levels.back().A.nrows;
-  NW_HIP(hipMalloc(&H.cinv, sizeof(double) * std::max<size_t>(h.coarse_inv.size(), 1)));
-  NW_HIP(hipMemcpyAsync(H.cinv, h.coarse_inv.data(), sizeof(double) * h.coarse_inv.size(),
+  std::vector<double> cinv(h.coarse_inv.begin(), h.coarse_inv.end());
+  if (nl == 1)  // solved directly: D A^-1, as the V-cycle returns
+    for (int64_t i = 0; i < H.nc; ++i) {
+      const double di = h.levels[0].dinv[i];
+      for (int64_t j = 0; j < H.nc; ++j) cinv[i * H.nc + j] *= di != 0.0 ? 1.0 / di : 0.0;
+    }
+  NW_HIP(hipMalloc(&H.cinv, sizeof(double) * std::max<size_t>(cinv.size(), 1)));
+  NW_HIP(hipMemcpyAsync(H.cinv, cinv.data(), sizeof(double) * cinv.size(),
                         hipMemcpyHostToDevice, st));
   NW_HIP(hipStreamSynchronize(st));
   H.ready = true;
@@ -548,22 +569,19 @@ static int narrow_hier(Ctx* c, const DevHier<double>& D, DevHier<float>& H)
     L.n = S.n;
     L.lmax = S.lmax;
     if (l == 0) {
+      L.A = DevMat<float>();
       L.A.n = S.A.n;
       L.A.sp = S.A.sp;
       L.A.ci = S.A.ci;
       L.A.dia_w = S.A.dia_w;
       L.A.dia_off = S.A.dia_off;
-      L.A.d16 = S.A.d16;
+      L.A.base = S.A.base;
       L.A.cd = S.A.cd;
       L.A.nv = S.A.nv;
-      NW_HIP(hipMalloc(&L.A.v, sizeof(float) * std::max<int64_t>(S.A.nv, 1)));
     } else {
       int rc = narrow_mat(S.A, L.A, st);
       if (rc) return rc;
     }
-    NW_HIP(hipMalloc(&L.dinv, sizeof(float) * std::max(L.n, 1)));
-    k_narrow<float><<<grid_for(L.n, kBlock), kBlock, 0, st>>>(S.dinv, L.dinv, L.n);
-    NW_LAUNCH_CHECK();
     int rc = alloc_level_vectors(L);
     if (!rc && l + 1 < nl) rc = narrow_mat(S.P, L.P, st);
     if (!rc && l + 1 < nl) rc = narrow_mat(S.R, L.R, st);
@@ -627,8 +645,8 @@ int amg_setup(Ctx* c, AmgDevice** out)
   const int rc = amg::build(std::move(A), o, h);
   NW_REQUIRE(rc == 0, NW_E_ARG, "AMG setup failed (%d): coarse level too "
              "large or singular", rc);
+  NW_REQUIRE(o.cheb_degree == 2, NW_E_ARG, "the V-cycle smooths with two Chebyshev terms");
   AmgDevice* a = new AmgDevice();
-  a->cheb_degree = o.cheb_degree;
   a->cheb_ratio = o.cheb_ratio;
   a->nlev = (int)h.levels.size();
   for (const auto& L : h.levels) {
@@ -637,19 +655,49 @@ int amg_setup(Ctx* c, AmgDevice** out)
   }
   int urc = upload_hier(c, h, a->d);
   // the smoothers' lambda_max(D^-1 A) on the device, every level but the
-  // coarsest (solved directly); the fine level's values first
-  if (!urc) {
-    DevLevel<double>& L0 = a->d.lv[0];
-    const Sell& sl = g.sell;
-    k_sell_values<double><<<grid_for(sl.len, kBlock), kBlock, 0, c->stream>>>(
-      sl.slot, sl.ci, g.vals, nullptr, L0.A.v, sl.len);
-    if (hipGetLastError() != hipSuccess) urc = NW_E_HIP;
-  }
-  for (int l = 0; !urc && l + 1 < a->nlev; ++l) {
+  // coarsest (solved directly), then the column scaling of the operators and
+  // prolongators (the coarsest level's iterate is x itself)
+  const int last = a->nlev - 1;
+  for (int l = 0; !urc && l < last; ++l) {
     DevLevel<double>& L = a->d.lv[l];
-    urc = device_lmax(L.n, L.x, L.t, L.dinv, [&](const double* x, double* y) {
-      mat_spmv<double>(L.A, x, y, 1.0, c->stream);
+    DevScratch tmp;
+    double* y = nullptr;
+    urc = tmp.alloc(&y, L.n);
+    if (l == 0 && !urc) {
+      const Sell& sl = g.sell;
+      double* v = nullptr;
+      urc = tmp.alloc(&v, sl.len);
+      if (!urc) {
+        k_sell_values<double><<<grid_for(sl.len, kBlock), kBlock, 0, c->stream>>>(
+          sl.slot, sl.ci, g.vals, nullptr, v, sl.len);
+        L.A.v = v;
+      }
+    }
+    if (urc) {
+      set_error("AMG setup: device allocation failed");
+      break;
+    }
+    urc = device_lmax(L.n, L.x, y, L.dinv, [&](const double* x, double* yv) {
+      mat_spmv<double>(L.A, x, yv, 1.0, c->stream);
     }, o.power_iters, c->stream, &L.lmax);
+    if (l == 0) L.A.v = nullptr;
+  }
+  for (int l = 0; !urc && l < last; ++l) {
+    DevLevel<double>& L = a->d.lv[l];
+    if (l > 0)
+      k_scale_mat<<<grid_for(L.n, kBlock), kBlock, 0, c->stream>>>(
+        L.A.sp, L.A.rp, L.A.ci, L.A.own_v, L.n, nullptr, L.dinv);
+    k_scale_mat<<<grid_for(L.n, kBlock), kBlock, 0, c->stream>>>(
+      L.P.sp, L.P.rp, L.P.ci, L.P.own_v, L.n, L.dinv,
+      l + 1 < last ? a->d.lv[l + 1].dinv : nullptr);
+    if (hipGetLastError() != hipSuccess) {
+      set_error("AMG setup: scaling kernel failed");
+      urc = NW_E_HIP;
+    }
+  }
+  if (!urc && hipStreamSynchronize(c->stream) != hipSuccess) {
+    set_error("AMG setup: device error");
+    urc = NW_E_HIP;
   }
   if (urc) {
     amg_free(a);
@@ -684,8 +732,10 @@ DevHier<float>& hier<float>(AmgDevice* a)
   return a->f;
 }
 
+const double* amg_fine_dinv(const AmgDevice* a) { return a->d.lv[0].dinv; }
+
 template <typename T>
-int amg_prepare(Ctx* c, AmgDevice* a, double* seconds)
+int amg_prepare(Ctx* c, AmgDevice* a, const T* fine, double* seconds)
 {
   DevHier<T>& H = hier<T>(a);
   NW_REQUIRE(a->d.ready, NW_E_STATE, "AMG hierarchy not set up");
@@ -699,71 +749,26 @@ int amg_prepare(Ctx* c, AmgDevice* a, double* seconds)
         *seconds = std::chrono::duration<double>(std::chrono::steady_clock::now() - t0).count();
     }
   }
-  // the fine level follows the current matrix values (sliced ELL order)
   const Sell& sl = c->g.sell;
   NW_REQUIRE(sl.ci && H.lv[0].A.ci == sl.ci, NW_E_STATE,
              "AMG fine level needs the graph's sliced ELL form");
-  k_sell_values<T><<<grid_for(sl.len, kBlock), kBlock, 0, c->stream>>>(
-    sl.slot, sl.ci, c->g.vals, nullptr, H.lv[0].A.v, sl.len);
-  NW_LAUNCH_CHECK();
+  H.lv[0].A.v = fine;
   return NW_OK;
 }
 
-// L.r = b - A x on level L
-template <typename T>
-static void level_resid(DevLevel<T>& L, const T* x, const T* b, hipStream_t st)
-{
-  mat_resid<T>(L.A, x, b, L.r, st);
-}
-
-// Chebyshev interval centre theta = (lmax + lmin) / 2 of level L
-static double cheb_theta(const AmgDevice* a, double lmax_est)
+// Two Chebyshev terms on [1.1 lmax / ratio, 1.1 lmax] from zero (Saad, Alg.
+// 12.1): z0 = v / theta, then d = c1 z0 + c2 (v - B z0) added to it.
+struct Smoother {
+  double alpha, beta;
+};
+static Smoother smoother(const AmgDevice* a, double lmax_est)
 {
   const double lmax = 1.1 * lmax_est, lmin = lmax / a->cheb_ratio;
-  return 0.5 * (lmax + lmin);
-}
-
-// z = p(D^-1 A) D^-1 b on level L (zero initial guess, degree k), written
-// to out, or with add added to out.  With init_done the first term
-// d = z = D^-1 b / theta is already in L.cd and L.cz (computed with the
-// residual b, mat_resid_cheb_init).
-template <typename T>
-static int cheb0(AmgDevice* a, DevLevel<T>& L, const T* b, T* out, bool add,
-                 bool init_done, hipStream_t st)
-{
-  const double lmax = 1.1 * L.lmax, lmin = lmax / a->cheb_ratio;
-  const double theta = cheb_theta(a, L.lmax), delta = 0.5 * (lmax - lmin);
-  const double sigma = theta / delta;
-  double rho = 1.0 / sigma;
-  const int k = a->cheb_degree;
-  if (!init_done) {
-    T* z0 = (k == 1 && !add) ? out : L.cz;
-    k_cheb_init<T><<<grid_for(L.n, kBlock), kBlock, 0, st>>>(
-      b, L.dinv, L.cd, z0, L.n, (T)(1.0 / theta));
-    NW_LAUNCH_CHECK();
-  }
-  NW_REQUIRE(k > 1 || !(add == false && init_done), NW_E_STATE,
-             "degree-1 smoother with a fused start");
-  if (k == 1) {
-    if (add) {
-      k_axpy_t<T><<<grid_for(L.n, kBlock), kBlock, 0, st>>>(out, L.cz, L.n);
-      NW_LAUNCH_CHECK();
-    }
-    return NW_OK;
-  }
-  T* z = L.cz;
-  T* z2 = L.cz2;
-  for (int it = 1; it < k; ++it) {
-    const double rho_new = 1.0 / (2.0 * sigma - rho);
-    const bool last = it == k - 1;
-    mat_cheb_step<T>(L.A, z, b, L.dinv, L.cd, last ? out : z2,
-                     (T)(rho_new * rho), (T)(2.0 * rho_new / delta),
-                     last && add, st);
-    NW_LAUNCH_CHECK();
-    std::swap(z, z2);
-    rho = rho_new;
-  }
-  return NW_OK;
+  const double theta = 0.5 * (lmax + lmin), delta = 0.5 * (lmax - lmin);
+  const double sigma = theta / delta, rho = 1.0 / sigma;
+  const double rho_new = 1.0 / (2.0 * sigma - rho);
+  const double c1 = rho_new * rho, c2 = 2.0 * rho_new / delta;
+  return {(1.0 + c1) / theta + c2, c2 / theta};
 }
 
 template <typename T>
@@ -773,29 +778,24 @@ static int vcycle(AmgDevice* a, DevHier<T>& H, int l, const T* b, T* x,
   DevLevel<T>& L = H.lv[l];
   const int last = (int)H.lv.size() - 1;
   if (l == last) {
-    if constexpr (sizeof(T) == 8)
-      k_dense_mv<<<grid_for(H.nc, 64), 64, 0, st>>>(H.cinv, H.nc, b, x);
-    else
-      k_dense_mv_f<<<grid_for(H.nc, 64), 64, 0, st>>>(H.cinv, H.nc, b, x);
+    k_dense_mv<T><<<grid_for((int64_t)H.nc * kWave, kBlock), kBlock, 0, st>>>(H.cinv, H.nc, b, x);
     NW_LAUNCH_CHECK();
     return NW_OK;
   }
   DevLevel<T>& C = H.lv[l + 1];
-  int rc = cheb0<T>(a, L, b, x, false, false, st);  // pre-smooth from zero
-  if (rc) return rc;
-  level_resid<T>(L, x, b, st);
-  NW_LAUNCH_CHECK();
+  const Smoother s = smoother(a, L.lmax);
+  mat_smooth<T>(L.A, b, x, (T)s.alpha, (T)s.beta, false, st);  // pre-smooth from zero
+  mat_resid<T>(L.A, x, b, L.r, st);
   mat_spmv<T>(L.R, L.r, C.b, (T)1, st);
   NW_LAUNCH_CHECK();
-  rc = vcycle<T>(a, H, l + 1, C.b, C.x, st);
+  const int rc = vcycle<T>(a, H, l + 1, C.b, C.x, st);
   if (rc) return rc;
   mat_spmv_add<T>(L.P, C.x, x, st);
-  NW_LAUNCH_CHECK();
   // post-smooth the correction of the new residual, added to x
-  mat_resid_cheb_init<T>(L.A, x, b, L.r, L.dinv, L.cd, L.cz,
-                         (T)(1.0 / cheb_theta(a, L.lmax)), st);
+  mat_resid<T>(L.A, x, b, L.r, st);
+  mat_smooth<T>(L.A, L.r, x, (T)s.alpha, (T)s.beta, true, st);
   NW_LAUNCH_CHECK();
-  return cheb0<T>(a, L, L.r, x, true, true, st);
+  return NW_OK;
 }
 
 template <typename T>
@@ -804,8 +804,8 @@ int amg_apply(AmgDevice* a, const T* b, T* x, hipStream_t st)
   return vcycle<T>(a, hier<T>(a), 0, b, x, st);
 }
 
-template int amg_prepare<double>(Ctx*, AmgDevice*, double*);
-template int amg_prepare<float>(Ctx*, AmgDevice*, double*);
+template int amg_prepare<double>(Ctx*, AmgDevice*, const double*, double*);
+template int amg_prepare<float>(Ctx*, AmgDevice*, const float*, double*);
 template int amg_apply<double>(AmgDevice*, const double*, double*, hipStream_t);
 template int amg_apply<float>(AmgDevice*, const float*, float*, hipStream_t);
 

@@ -27,7 +27,7 @@
 // are reproducible run to run.
 //
 // Preconditioners (right): Jacobi, applied by scaling the matrix columns
-// once per solve (A D^-1); Chebyshev of degree k on D^-1 A over
+// once per solve (A D^-1, which the AMG V-cycle works on as well); Chebyshev of degree k on D^-1 A over
 // [lmax/ratio, lmax] (Saad, Iterative Methods for Sparse Linear Systems,
 // 2nd ed., Alg. 12.1), lmax from a seeded power iteration.
 #include <algorithm>
@@ -642,41 +642,51 @@ __global__ __launch_bounds__(kBlock) void k_sell_struct(
   }
 }
 
-// The delta form of each slice not in offset form (a wave per slice):
-// when every column of its rows lies within 32767 of the row, cd[p] =
-// column - row and d16[k] = 1; else d16[k] = 0.
+// The delta form of each slice not in offset form (a wave per slice): when
+// its columns span less than 65536, base[k] = the smallest and cd[p] = column
+// - base; else base[k] = -1.
 __global__ __launch_bounds__(kBlock) void k_sell_delta16(
-  const int64_t* __restrict__ sp, const int32_t* __restrict__ sci, int n, int nslices,
-  const int32_t* __restrict__ dia_w, int16_t* __restrict__ cd, int8_t* __restrict__ d16)
+  const int64_t* __restrict__ sp, const int32_t* __restrict__ sci, int nslices,
+  const int32_t* __restrict__ dia_w, uint16_t* __restrict__ cd, int32_t* __restrict__ base)
 {
   const int t = blockIdx.x * blockDim.x + threadIdx.x;
   const int k = t >> 6;
   if (k >= nslices) return;  // whole waves
   const int64_t b = sp[k] + (t & 63);
   const int w = (int)((sp[k + 1] - sp[k]) >> 6);
-  bool fits = true;
-  for (int j = 0; j < w && t < n; ++j) {
-    const int d = sci[b + 64 * (int64_t)j] - t;
-    fits = fits && d >= -32767 && d <= 32767;
+  int lo = INT_MAX, hi = 0;
+  for (int j = 0; j < w; ++j) {
+    const int c = sci[b + 64 * (int64_t)j];
+    lo = min(lo, c);
+    hi = max(hi, c);
   }
-  const bool ok = (dia_w == nullptr || dia_w[k] == 0) && __ballot(!fits) == 0;
+  for (int o = kWave / 2; o > 0; o >>= 1) {
+    lo = min(lo, __shfl_xor(lo, o, kWave));
+    hi = max(hi, __shfl_xor(hi, o, kWave));
+  }
+  const bool ok = w > 0 && (dia_w == nullptr || dia_w[k] == 0) && hi - lo < 65536;
   for (int j = 0; j < w; ++j) {
     const int64_t p = b + 64 * (int64_t)j;
-    cd[p] = ok && t < n ? (int16_t)(sci[p] - t) : (int16_t)0;
+    cd[p] = ok ? (uint16_t)(sci[p] - lo) : (uint16_t)0;
   }
-  if ((t & 63) == 0) d16[k] = ok ? 1 : 0;
+  if ((t & 63) == 0) base[k] = ok ? lo : -1;
 }
 
 }  // namespace
+
+void sell_free(Sell& s)
+{
+  for (void* p : {(void*)s.sp, (void*)s.ci, (void*)s.slot, (void*)s.dia_w, (void*)s.dia_off,
+                  (void*)s.base, (void*)s.cd})
+    (void)hipFree(p);
+  s = Sell();
+}
 
 int sell_build(const int32_t* rp, const int32_t* ci, int n, Sell& s,
                hipStream_t st, bool pad_last, bool offsets)
 {
   // the callers pass a new structure or one a failed build left part way
-  for (void* p : {(void*)s.sp, (void*)s.ci, (void*)s.slot, (void*)s.dia_w, (void*)s.dia_off,
-                  (void*)s.d16, (void*)s.cd})
-    (void)hipFree(p);
-  s = Sell();
+  sell_free(s);
   s.n = n;
   s.nslices = (n + kWave - 1) / kWave;
   const int ns = s.nslices;
@@ -723,22 +733,20 @@ int sell_build(const int32_t* rp, const int32_t* ci, int n, Sell& s,
   k_sell_struct<<<grid, kBlock, 0, st>>>(rp, ci, n, s.sp, ns, s.ci, s.slot, pad_last,
                                          s.dia_w, s.dia_off);
   NW_LAUNCH_CHECK();
-  if (offsets) {
-    NW_HIP(hipMalloc(&s.d16, sizeof(int8_t) * std::max(ns, 1)));
-    NW_HIP(hipMalloc(&s.cd, sizeof(int16_t) * std::max<int64_t>(s.len, 1)));
-    k_sell_delta16<<<grid, kBlock, 0, st>>>(s.sp, s.ci, n, ns, s.dia_w, s.cd, s.d16);
-    NW_LAUNCH_CHECK();
-    std::vector<int8_t> d16(ns);
-    NW_HIP(hipMemcpyAsync(d16.data(), s.d16, ns, hipMemcpyDeviceToHost, st));
-    NW_HIP(hipStreamSynchronize(st));
-    s.d16_slices = 0;
-    for (int k = 0; k < ns; ++k) s.d16_slices += d16[k];
-    if (s.d16_slices == 0) {  // nothing to gain
-      (void)hipFree(s.d16);
-      (void)hipFree(s.cd);
-      s.d16 = nullptr;
-      s.cd = nullptr;
-    }
+  NW_HIP(hipMalloc(&s.base, sizeof(int32_t) * std::max(ns, 1)));
+  NW_HIP(hipMalloc(&s.cd, sizeof(uint16_t) * std::max<int64_t>(s.len, 1)));
+  k_sell_delta16<<<grid, kBlock, 0, st>>>(s.sp, s.ci, ns, s.dia_w, s.cd, s.base);
+  NW_LAUNCH_CHECK();
+  std::vector<int32_t> base(ns);
+  NW_HIP(hipMemcpyAsync(base.data(), s.base, sizeof(int32_t) * ns, hipMemcpyDeviceToHost, st));
+  NW_HIP(hipStreamSynchronize(st));
+  s.delta_slices = 0;
+  for (int k = 0; k < ns; ++k) s.delta_slices += base[k] >= 0;
+  if (s.delta_slices == 0) {  // nothing to gain
+    (void)hipFree(s.base);
+    (void)hipFree(s.cd);
+    s.base = nullptr;
+    s.cd = nullptr;
   }
   NW_HIP(hipStreamSynchronize(st));
   return NW_OK;
@@ -814,14 +822,14 @@ void free_krylov(Krylov* k)
 }
 
 template <typename T>
-static int alloc_space(Space<T>& s, int64_t n, int64_t nnz, int m, bool cheb)
+static int alloc_space(Space<T>& s, int64_t n, int64_t nnz, int m, bool cheb, bool amg)
 {
   if (!s.V) NW_HIP(hipMalloc(&s.V, sizeof(T) * n * (m + 1)));
   if (!s.mat) NW_HIP(hipMalloc(&s.mat, sizeof(T) * nnz));  // sliced ELL order
   if (!s.u) NW_HIP(hipMalloc(&s.u, sizeof(T) * n));
+  if ((cheb || amg) && !s.cz) NW_HIP(hipMalloc(&s.cz, sizeof(T) * n));
   if (cheb) {
     if (!s.dinv) NW_HIP(hipMalloc(&s.dinv, sizeof(T) * n));
-    if (!s.cz) NW_HIP(hipMalloc(&s.cz, sizeof(T) * n));
     if (!s.cd) NW_HIP(hipMalloc(&s.cd, sizeof(T) * n));
     if (!s.cz2) NW_HIP(hipMalloc(&s.cz2, sizeof(T) * n));
   }
@@ -908,7 +916,8 @@ struct Solve {
     return NW_OK;
   }
 
-  // W = A M^-1 v
+  // W = A M^-1 v (under AMG as (A D^-1) (D M^-1 v): the V-cycle works on
+  // column-scaled operators and returns D M^-1 v)
   template <typename T>
   int apply_op(Space<T>& s, const T* v, T* W)
   {
@@ -1095,8 +1104,11 @@ struct Solve {
       if (rc) return rc;
       u = s.cz;
     }
-    k_axpy_prec<T><<<grid_for(n, kBlock), kBlock, 0, st>>>(
-      x, u, cfg->precond == NW_PREC_JACOBI ? k->dinv : nullptr, n);
+    // under Jacobi and AMG u is D M^-1 Q y, the iterate of A D^-1
+    const double* dinv = cfg->precond == NW_PREC_JACOBI ? k->dinv
+                         : cfg->precond == NW_PREC_AMG  ? amg_fine_dinv(c->amg)
+                                                        : nullptr;
+    k_axpy_prec<T><<<grid_for(n, kBlock), kBlock, 0, st>>>(x, u, dinv, n);
     NW_LAUNCH_CHECK();
     return NW_OK;
   }
@@ -1215,8 +1227,8 @@ int nw_linsys_solve(nw_ctx* c, const nw_solver_cfg* cfg, nw_solve_stats* out)
     if (rc0) return rc0;
   }
   const int64_t slen = c->g.sell.len;
-  int rc = f32 ? alloc_space(k->f, n, slen, k->m, cheb || amgp)
-               : alloc_space(k->d, n, slen, k->m, cheb || amgp);
+  int rc = f32 ? alloc_space(k->f, n, slen, k->m, cheb, amgp)
+               : alloc_space(k->d, n, slen, k->m, cheb, amgp);
   if (rc) return rc;
   if (cheb && !k->pe) NW_HIP(hipMalloc(&k->pe, sizeof(double) * 2 * n));
 
@@ -1229,8 +1241,10 @@ int nw_linsys_solve(nw_ctx* c, const nw_solver_cfg* cfg, nw_solve_stats* out)
     out->setup_ms = 1e3 * amg_setup_seconds(c->amg);
   }
   if (amgp) {
+    // the cycle's matrix copy is the V-cycle's fine level
     double narrow_s = 0.0;  // the FP32 hierarchy, made on first use
-    rc = f32 ? amg_prepare<float>(c, c->amg, &narrow_s) : amg_prepare<double>(c, c->amg);
+    rc = f32 ? amg_prepare<float>(c, c->amg, k->f.mat, &narrow_s)
+             : amg_prepare<double>(c, c->amg, k->d.mat);
     if (rc) return rc;
     out->setup_ms += 1e3 * narrow_s;
     out->precond_levels = amg_levels(c->amg);
@@ -1247,7 +1261,9 @@ int nw_linsys_solve(nw_ctx* c, const nw_solver_cfg* cfg, nw_solve_stats* out)
   NW_HIP(hipMemcpyAsync(&bad, k->bad, sizeof(int), hipMemcpyDeviceToHost, st));
   NW_HIP(hipStreamSynchronize(st));
   NW_REQUIRE(!bad, NW_E_NONFINITE, "zero or non-finite diagonal in the matrix");
-  const double* colscale = (cfg->precond == NW_PREC_JACOBI) ? k->dinv : nullptr;
+  const double* colscale = cfg->precond == NW_PREC_JACOBI ? k->dinv
+                           : amgp                         ? amg_fine_dinv(c->amg)
+                                                          : nullptr;
   const Sell& sl = c->g.sell;
   if (f32) {
     k_sell_values<float><<<grid_for(sl.len, kBlock), kBlock, 0, st>>>(

@@ -78,27 +78,23 @@ __global__ void k_cheb_init(const T* __restrict__ v, const T* __restrict__ dinv,
   z[i] = di;
 }
 
-// Chebyshev step: r = v - A z; d = c1 d + c2 dinv r; zo = z + d (with ADD,
-// zo += z + d: the last step of a smoother that corrects zo).
+// Two Chebyshev terms on v from zero, with A's columns scaled to a unit
+// diagonal: out = alpha v - beta A v (with ADD added to out); see
+// AmgDevice in nw_amg.hip.
 template <typename T, int G, bool ADD = false>
-__global__ __launch_bounds__(kBlock) void k_cheb_step(
+__global__ __launch_bounds__(kBlock) void k_smooth(
   const int32_t* __restrict__ rp, const int32_t* __restrict__ ci,
-  const T* __restrict__ va, const T* __restrict__ z, const T* __restrict__ v,
-  const T* __restrict__ dinv, T* __restrict__ d, T* __restrict__ zo, int n,
-  T c1, T c2)
+  const T* __restrict__ va, const T* __restrict__ v, T* __restrict__ out, int n,
+  T alpha, T beta)
 {
   const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   const int row = (int)(t / G);
   const int g = threadIdx.x & (G - 1);
-  T s = row < n ? csr_dot<T, G>(rp, ci, va, z, row, g) : (T)0;
+  T s = row < n ? csr_dot<T, G>(rp, ci, va, v, row, g) : (T)0;
   for (int o = G / 2; o > 0; o >>= 1) s += __shfl_xor(s, o, G);
   if (row < n && g == 0) {
-    const T dn = c1 * d[row] + c2 * dinv[row] * (v[row] - s);
-    d[row] = dn;
-    if (ADD)
-      zo[row] += z[row] + dn;
-    else
-      zo[row] = z[row] + dn;
+    const T e = alpha * v[row] - beta * s;
+    out[row] = ADD ? out[row] + e : e;
   }
 }
 
@@ -131,29 +127,6 @@ __global__ __launch_bounds__(kBlock) void k_resid(
   if (row < n && g == 0) r[row] = b[row] - s;
 }
 
-// r = b - A x, and the start of a Chebyshev smoother on r:
-// d = z = dinv r inv_theta (k_resid followed by k_cheb_init).
-template <typename T, int G>
-__global__ __launch_bounds__(kBlock) void k_resid_cheb_init(
-  const int32_t* __restrict__ rp, const int32_t* __restrict__ ci,
-  const T* __restrict__ va, const T* __restrict__ x, const T* __restrict__ b,
-  T* __restrict__ r, const T* __restrict__ dinv, T* __restrict__ d,
-  T* __restrict__ z, int n, T inv_theta)
-{
-  const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  const int row = (int)(t / G);
-  const int g = threadIdx.x & (G - 1);
-  T s = row < n ? csr_dot<T, G>(rp, ci, va, x, row, g) : (T)0;
-  for (int o = G / 2; o > 0; o >>= 1) s += __shfl_xor(s, o, G);
-  if (row < n && g == 0) {
-    const T ri = b[row] - s;
-    r[row] = ri;
-    const T di = dinv[row] * ri * inv_theta;
-    d[row] = di;
-    z[row] = di;
-  }
-}
-
 // ------------------------------------------------------------ sliced ELL
 // One lane per row, a wave per slice: for every j the 64 lanes read 64
 // consecutive values and columns, and all loads of a row are independent
@@ -162,8 +135,8 @@ __global__ __launch_bounds__(kBlock) void k_resid_cheb_init(
 // column with value 0.  The row sum runs over j in order.  A slice in
 // offset form (A.dia_w[k] > 0) takes its columns as row + the slice's
 // offsets, which are the same for the whole wave (scalar loads), and reads
-// no column array; a slice in delta form (A.d16[k]) reads 16-bit column -
-// row deltas instead of the 32-bit columns.
+// no column array; a slice in delta form (A.base[k] >= 0) reads 16-bit
+// columns relative to its base instead of the 32-bit columns.
 template <typename T>
 __device__ inline T sell_dot(const SellView& A, const T* __restrict__ va,
                              const T* __restrict__ x, int row)
@@ -189,14 +162,15 @@ __device__ inline T sell_dot(const SellView& A, const T* __restrict__ va,
     }
     return s;
   }
-  if (A.d16 && A.d16[k]) {
+  const int base = A.base ? A.base[k] : -1;
+  if (base >= 0) {
     for (int j0 = 0; j0 < w; j0 += 8) {
       int c[8];
       T v[8];
 #pragma unroll
       for (int u = 0; u < 8; ++u) {
         const int j = min(j0 + u, w - 1);
-        c[u] = row + A.cd[b + 64 * (int64_t)j];
+        c[u] = base + A.cd[b + 64 * (int64_t)j];
         v[u] = j0 + u < w ? va[b + 64 * (int64_t)j] : (T)0;
       }
 #pragma unroll
@@ -240,9 +214,8 @@ __global__ __launch_bounds__(kBlock) void k_sell_spmv_add(
   y[row] += sell_dot(A, va, x, row);
 }
 
-// Chebyshev step: r = v - A z; d = c1 d + c2 dinv r; zo = z + d (with ADD,
-// zo += z + d).
-template <typename T, bool ADD = false>
+// Chebyshev step: r = v - A z; d = c1 d + c2 dinv r; zo = z + d.
+template <typename T>
 __global__ __launch_bounds__(kBlock) void k_sell_cheb_step(
   SellView A, const T* __restrict__ va, const T* __restrict__ z, const T* __restrict__ v,
   const T* __restrict__ dinv, T* __restrict__ d, T* __restrict__ zo, int n,
@@ -253,10 +226,19 @@ __global__ __launch_bounds__(kBlock) void k_sell_cheb_step(
   const T s = sell_dot(A, va, z, row);
   const T dn = c1 * d[row] + c2 * dinv[row] * (v[row] - s);
   d[row] = dn;
-  if (ADD)
-    zo[row] += z[row] + dn;
-  else
-    zo[row] = z[row] + dn;
+  zo[row] = z[row] + dn;
+}
+
+// out = alpha v - beta A v, with ADD added to out (k_smooth)
+template <typename T, bool ADD = false>
+__global__ __launch_bounds__(kBlock) void k_sell_smooth(
+  SellView A, const T* __restrict__ va, const T* __restrict__ v, T* __restrict__ out, int n,
+  T alpha, T beta)
+{
+  const int row = blockIdx.x * blockDim.x + threadIdx.x;
+  if (row >= n) return;
+  const T e = alpha * v[row] - beta * sell_dot(A, va, v, row);
+  out[row] = ADD ? out[row] + e : e;
 }
 
 // r = b - A x
@@ -268,22 +250,6 @@ __global__ __launch_bounds__(kBlock) void k_sell_resid(
   const int row = blockIdx.x * blockDim.x + threadIdx.x;
   if (row >= n) return;
   r[row] = b[row] - sell_dot(A, va, x, row);
-}
-
-// r = b - A x and d = z = dinv r inv_theta (k_sell_resid + k_cheb_init)
-template <typename T>
-__global__ __launch_bounds__(kBlock) void k_sell_resid_cheb_init(
-  SellView A, const T* __restrict__ va, const T* __restrict__ x, const T* __restrict__ b,
-  T* __restrict__ r, const T* __restrict__ dinv, T* __restrict__ d,
-  T* __restrict__ z, int n, T inv_theta)
-{
-  const int row = blockIdx.x * blockDim.x + threadIdx.x;
-  if (row >= n) return;
-  const T ri = b[row] - sell_dot(A, va, x, row);
-  r[row] = ri;
-  const T di = dinv[row] * ri * inv_theta;
-  d[row] = di;
-  z[row] = di;
 }
 
 // out[p] = T(a[slot[p]] * (colscale ? colscale[ci[p]] : 1)), 0 for padding
@@ -305,15 +271,15 @@ __global__ void k_sell_values(const int32_t* __restrict__ slot,
 // arrays are released first).  Padding positions read the row's own index as column
 // (square matrices), or with pad_last the row's last column, which keeps
 // them inside the columns of a rectangular matrix.  With offsets (square
-// matrices only) the slices that qualify are stored in offset form, and
-// the others whose columns lie within 32767 of their rows get 16-bit
-// deltas.
+// matrices only) the slices that qualify are stored in offset form; the
+// others whose columns span less than 65536 get 16-bit ones.
 int sell_build(const int32_t* rp, const int32_t* ci, int n, Sell& s,
                hipStream_t st, bool pad_last = false, bool offsets = false);
+void sell_free(Sell& s);
 
 inline SellView sell_view(const Sell& s)
 {
-  return {s.sp, s.ci, s.dia_w, s.dia_off, s.d16, s.cd};
+  return {s.sp, s.ci, s.dia_w, s.dia_off, s.base, s.cd};
 }
 
 // launch helper: dispatch a G-templated row kernel by lanes-per-row

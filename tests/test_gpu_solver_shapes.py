@@ -72,3 +72,33 @@ def test_exhausted_krylov_space(nw, ctx):
     xd = orc.dense_solve(A.dense(), A.rhs)
     assert st.converged and st.iters <= 8
     np.testing.assert_allclose(ctx.solution(), xd, rtol=0, atol=1e-9 * np.abs(xd).max())
+
+
+@pytest.mark.parametrize("shape", [(4, 2, 2), (10, 9, 8), (11, 10, 9), (22, 21, 20)])
+@pytest.mark.parametrize("mode", [0, 1])
+def test_amg_levels(nw, ctx, shape, mode):
+    """One level (solved directly), just below and above the direct solve's
+    size, and several levels, the hierarchy reused for another matrix (its
+    diagonal then is not the one the columns are scaled by)."""
+    P, A = _system(nw, ctx, shape)
+    tol = 1e-10 if mode == 0 else 1e-8
+    cfg = nw.solver_cfg(kspace=30, max_iters=300, tol=tol, precond=nw.PREC_AMG, mode=mode,
+                        inner_tol=1e-4, reuse_preconditioner=0)
+    st = ctx.solve(cfg)
+    levels = ctx.amg_levels()
+    assert len(levels) == st.precond_levels
+    if P.n <= 1000:
+        assert st.precond_levels == 1 and st.iters <= (2 if mode == 0 else 6)
+    r = A.rhs - A.spmv(ctx.solution())
+    assert st.converged and np.linalg.norm(r) <= 1.0001 * tol * np.linalg.norm(A.rhs)
+    # another time step, near enough for the smoothers' intervals
+    o = nw.continuity_defaults(dt=0.95)
+    ctx.assemble_continuity(o)
+    top = np.where(np.abs(P.coords[:, 2] - 1.0) < 1e-12)[0].astype(np.int32)
+    ctx.apply_dirichlet(top, nw.F_PRESSURE, nw.F_DIFF_FLUX_COEFF, 0, 1)
+    cfg.reuse_preconditioner = 1
+    s2 = ctx.solve(cfg)
+    B = P.oracle_continuity(pb.to_orc_continuity(o))
+    B.apply_dirichlet(top, 0, 1, P.p, np.zeros(P.n))
+    r = B.rhs - B.spmv(ctx.solution())
+    assert s2.converged and np.linalg.norm(r) <= 1.0001 * tol * np.linalg.norm(B.rhs)
