@@ -78,13 +78,13 @@ __global__ __launch_bounds__(kBlock) void k_scale_mat(
 }  // namespace
 
 // A level operator, in sliced ELL form (sp != nullptr: the layout of Sell,
-// one lane per row) when its rows are short, else in CSR with G lanes per
+// G = 1 or 2 lanes per row) when its rows are short, else in CSR with G lanes per
 // row (rp).  The fine-level A uses the graph's sliced ELL structure; the
 // others own theirs.
 template <typename T>
 struct DevMat {
   int n = 0;  // rows
-  int G = 8;
+  int G = 1;  // lanes per row
   const int64_t* sp = nullptr;
   const int32_t* rp = nullptr;
   const int32_t* ci = nullptr;
@@ -112,8 +112,7 @@ static void mat_spmv(const DevMat<T>& M, const T* x, T* y, T alpha,
                      hipStream_t st)
 {
   if (M.sp)
-    k_sell_spmv<T><<<grid_for(M.n, kBlock), kBlock, 0, st>>>(M.view(), M.v, x, y, M.n,
-                                                             alpha);
+    NW_SELL_LAUNCH(k_sell_spmv, T, M.G, M.n, st, M.view(), M.v, x, y, M.n, alpha);
   else
     NW_ROW_LAUNCH(k_spmv, T, M.G, M.n, st, M.rp, M.ci, M.v, x, y, M.n, alpha);
 }
@@ -122,8 +121,7 @@ template <typename T>
 static void mat_spmv_add(const DevMat<T>& M, const T* x, T* y, hipStream_t st)
 {
   if (M.sp)
-    k_sell_spmv_add<T><<<grid_for(M.n, kBlock), kBlock, 0, st>>>(M.view(), M.v, x, y,
-                                                                 M.n);
+    NW_SELL_LAUNCH(k_sell_spmv_add, T, M.G, M.n, st, M.view(), M.v, x, y, M.n);
   else
     NW_ROW_LAUNCH(k_spmv_add, T, M.G, M.n, st, M.rp, M.ci, M.v, x, y, M.n);
 }
@@ -133,8 +131,7 @@ static void mat_resid(const DevMat<T>& M, const T* x, const T* b, T* r,
                       hipStream_t st)
 {
   if (M.sp)
-    k_sell_resid<T><<<grid_for(M.n, kBlock), kBlock, 0, st>>>(M.view(), M.v, x, b, r,
-                                                              M.n);
+    NW_SELL_LAUNCH(k_sell_resid, T, M.G, M.n, st, M.view(), M.v, x, b, r, M.n);
   else
     NW_ROW_LAUNCH(k_resid, T, M.G, M.n, st, M.rp, M.ci, M.v, x, b, r, M.n);
 }
@@ -145,11 +142,9 @@ static void mat_smooth(const DevMat<T>& M, const T* v, T* out, T alpha, T beta, 
                        hipStream_t st)
 {
   if (M.sp && add)
-    k_sell_smooth<T, true><<<grid_for(M.n, kBlock), kBlock, 0, st>>>(M.view(), M.v, v, out,
-                                                                     M.n, alpha, beta);
+    NW_SELL_LAUNCH_ADD(k_sell_smooth, T, M.G, M.n, st, M.view(), M.v, v, out, M.n, alpha, beta);
   else if (M.sp)
-    k_sell_smooth<T><<<grid_for(M.n, kBlock), kBlock, 0, st>>>(M.view(), M.v, v, out, M.n,
-                                                               alpha, beta);
+    NW_SELL_LAUNCH(k_sell_smooth, T, M.G, M.n, st, M.view(), M.v, v, out, M.n, alpha, beta);
   else if (add)
     NW_ROW_LAUNCH_ADD(k_smooth, T, M.G, M.n, st, M.rp, M.ci, M.v, v, out, M.n, alpha, beta);
   else
@@ -459,6 +454,7 @@ static int upload_mat(const amg::Csr& h, DevMat<double>& d, hipStream_t st)
   Sell& s = d.own;  // owned by d, also after a failure
   rc = sell_build(drp, dci, (int)n, s, st, true);
   if (rc) return rc;
+  d.G = sell_lanes(n, avg);
   d.sp = s.sp;
   d.ci = s.ci;
   d.base = s.base;

@@ -863,7 +863,7 @@ struct Solve {
   int spmv(const T* va, const T* x, T* y, T alpha)
   {
     const int n = (int)k->n;
-    k_sell_spmv<T><<<grid_for(n, kBlock), kBlock, 0, st>>>(
+    k_sell_spmv<T, 1><<<grid_for(n, kBlock), kBlock, 0, st>>>(
       sell_view(c->g.sell), va, x, y, n, alpha);
     NW_LAUNCH_CHECK();
     return NW_OK;

@@ -10,6 +10,9 @@
 
 namespace nw {
 
+// rows a one-lane-per-row kernel needs to fill the chip: 64 waves per CU
+constexpr int64_t kSellFillRows = 256 * 64 * 64;
+
 // Lanes per row for CSR rows of `avg` entries: each lane takes kCsrUnroll
 // entries per step as independent loads, so a row of average length is
 // covered by about one step (measured on the 20-entry AMG coarse operator
@@ -128,90 +131,97 @@ __global__ __launch_bounds__(kBlock) void k_resid(
 }
 
 // ------------------------------------------------------------ sliced ELL
-// One lane per row, a wave per slice: for every j the 64 lanes read 64
-// consecutive values and columns, and all loads of a row are independent
-// (issued eight at a time), so a wave keeps a whole row's gathers in
-// flight instead of walking a dependent chain.  Padding reads x at a valid
-// column with value 0.  The row sum runs over j in order.  A slice in
+// G lanes per row (sell_lanes): a wave takes 64 / G consecutive rows of a
+// slice, lane l the entries j = l / (64 / G) mod G of row l % (64 / G), so
+// that for every j the lanes read consecutive values and columns; all loads
+// of a lane are independent (issued eight at a time), and a wave keeps its
+// rows' gathers in flight instead of walking a dependent chain.  Padding
+// reads x at a valid column with value 0.  With one lane the row sum runs
+// over j in order; G lanes' sums are added by a fixed butterfly.  A slice in
 // offset form (A.dia_w[k] > 0) takes its columns as row + the slice's
-// offsets, which are the same for the whole wave (scalar loads), and reads
-// no column array; a slice in delta form (A.base[k] >= 0) reads 16-bit
-// columns relative to its base instead of the 32-bit columns.
-template <typename T>
-__device__ inline T sell_dot(const SellView& A, const T* __restrict__ va,
-                             const T* __restrict__ x, int row)
+// offsets, which are the same for the whole wave (scalar loads with one
+// lane), and reads no column array; a slice in delta form (A.base[k] >= 0)
+// reads 16-bit columns relative to its base instead of the 32-bit columns.
+struct SellLane {
+  int row, g;
+};
+template <int G>
+__device__ inline SellLane sell_lane()
 {
-  // rows of one slice are one wave: the slice index is wave-uniform
+  constexpr int R = kWave / G;
+  const int t = blockIdx.x * kBlock + threadIdx.x;
+  const int lane = t & (kWave - 1);
+  return {(t / kWave) * R + lane % R, lane / R};
+}
+
+template <typename T, int G>
+__device__ inline T sell_dot(const SellView& A, const T* __restrict__ va,
+                             const T* __restrict__ x, SellLane l)
+{
+  // rows of one wave are in one slice: the slice index is wave-uniform
+  const int row = l.row;
   const int k = __builtin_amdgcn_readfirstlane(row >> 6);
   const int64_t b = A.sp[k] + (row & 63);
   const int w = (int)((A.sp[k + 1] - A.sp[k]) >> 6);
   T s = 0;
+  auto sum = [&](auto column) {
+    for (int j0 = l.g; j0 < w; j0 += 8 * G) {
+      int c[8];
+      T v[8];
+#pragma unroll
+      for (int u = 0; u < 8; ++u) {
+        const int j = min(j0 + u * G, w - 1);
+        c[u] = column(j);
+        v[u] = j0 + u * G < w ? va[b + 64 * (int64_t)j] : (T)0;
+      }
+#pragma unroll
+      for (int u = 0; u < 8; ++u) s += v[u] * x[c[u]];
+    }
+  };
+  const int base = A.base ? A.base[k] : -1;
   if (A.dia_w && A.dia_w[k] > 0) {
     const int32_t* off = A.dia_off + (int64_t)k * kDiaMax;
-    for (int j0 = 0; j0 < w; j0 += 8) {
-      int c[8];
-      T v[8];
-#pragma unroll
-      for (int u = 0; u < 8; ++u) {
-        const int j = min(j0 + u, w - 1);
-        c[u] = row + off[j];
-        v[u] = j0 + u < w ? va[b + 64 * (int64_t)j] : (T)0;
-      }
-#pragma unroll
-      for (int u = 0; u < 8; ++u) s += v[u] * x[c[u]];
-    }
-    return s;
+    sum([&](int j) { return row + off[j]; });
+  } else if (base >= 0) {
+    sum([&](int j) { return base + A.cd[b + 64 * (int64_t)j]; });
+  } else {
+    sum([&](int j) { return A.ci[b + 64 * (int64_t)j]; });
   }
-  const int base = A.base ? A.base[k] : -1;
-  if (base >= 0) {
-    for (int j0 = 0; j0 < w; j0 += 8) {
-      int c[8];
-      T v[8];
-#pragma unroll
-      for (int u = 0; u < 8; ++u) {
-        const int j = min(j0 + u, w - 1);
-        c[u] = base + A.cd[b + 64 * (int64_t)j];
-        v[u] = j0 + u < w ? va[b + 64 * (int64_t)j] : (T)0;
-      }
-#pragma unroll
-      for (int u = 0; u < 8; ++u) s += v[u] * x[c[u]];
-    }
-    return s;
-  }
-  for (int j0 = 0; j0 < w; j0 += 8) {
-    int c[8];
-    T v[8];
-#pragma unroll
-    for (int u = 0; u < 8; ++u) {
-      const int j = min(j0 + u, w - 1);
-      c[u] = A.ci[b + 64 * (int64_t)j];
-      v[u] = j0 + u < w ? va[b + 64 * (int64_t)j] : (T)0;
-    }
-#pragma unroll
-    for (int u = 0; u < 8; ++u) s += v[u] * x[c[u]];
-  }
+  for (int o = kWave / G; o < kWave; o *= 2) s += __shfl_xor(s, o);
   return s;
 }
 
+// Lanes per row of a sliced ELL matrix of n rows, `avg` entries on average:
+// one where its waves fill the chip by themselves or its rows are too short
+// to share, else two (level 1 of the 0.96 M-row box, 207 thousand rows of 20
+// entries, FP64: 12.5 us with two lanes, 13.9 with one, 13.0 with four; of the
+// 4.2 M-row one, 933 thousand rows, FP32: 27 against 28 us).
+inline int sell_lanes(int64_t n, double avg)
+{
+  return n < kSellFillRows && avg >= 8.0 ? 2 : 1;
+}
+
 // y = alpha * (A x)
-template <typename T>
+template <typename T, int G>
 __global__ __launch_bounds__(kBlock) void k_sell_spmv(
   SellView A, const T* __restrict__ va, const T* __restrict__ x, T* __restrict__ y, int n,
   T alpha)
 {
-  const int row = blockIdx.x * blockDim.x + threadIdx.x;
-  if (row >= n) return;
-  y[row] = alpha * sell_dot(A, va, x, row);
+  const SellLane l = sell_lane<G>();
+  if (l.row - l.row % (kWave / G) >= n) return;  // whole waves
+  const T s = sell_dot<T, G>(A, va, x, l);
+  if (l.row < n && l.g == 0) y[l.row] = alpha * s;
 }
 
 // y += A x
-template <typename T>
+template <typename T, int G>
 __global__ __launch_bounds__(kBlock) void k_sell_spmv_add(
   SellView A, const T* __restrict__ va, const T* __restrict__ x, T* __restrict__ y, int n)
 {
-  const int row = blockIdx.x * blockDim.x + threadIdx.x;
-  if (row >= n) return;
-  y[row] += sell_dot(A, va, x, row);
+  const SellLane l = sell_lane<G>();
+  if (l.row - l.row % (kWave / G) >= n) return;
+  const T s = sell_dot<T, G>(A, va, x, l);
+  if (l.row < n && l.g == 0) y[l.row] += s;
 }
 
 // Chebyshev step: r = v - A z; d = c1 d + c2 dinv r; zo = z + d.
@@ -221,35 +231,41 @@ __global__ __launch_bounds__(kBlock) void k_sell_cheb_step(
   const T* __restrict__ dinv, T* __restrict__ d, T* __restrict__ zo, int n,
   T c1, T c2)
 {
-  const int row = blockIdx.x * blockDim.x + threadIdx.x;
+  const SellLane l = sell_lane<1>();
+  const int row = l.row;
   if (row >= n) return;
-  const T s = sell_dot(A, va, z, row);
+  const T s = sell_dot<T, 1>(A, va, z, l);
   const T dn = c1 * d[row] + c2 * dinv[row] * (v[row] - s);
   d[row] = dn;
   zo[row] = z[row] + dn;
 }
 
 // out = alpha v - beta A v, with ADD added to out (k_smooth)
-template <typename T, bool ADD = false>
+template <typename T, int G, bool ADD = false>
 __global__ __launch_bounds__(kBlock) void k_sell_smooth(
   SellView A, const T* __restrict__ va, const T* __restrict__ v, T* __restrict__ out, int n,
   T alpha, T beta)
 {
-  const int row = blockIdx.x * blockDim.x + threadIdx.x;
-  if (row >= n) return;
-  const T e = alpha * v[row] - beta * sell_dot(A, va, v, row);
-  out[row] = ADD ? out[row] + e : e;
+  const SellLane l = sell_lane<G>();
+  const int row = l.row;
+  if (row - row % (kWave / G) >= n) return;
+  const T s = sell_dot<T, G>(A, va, v, l);
+  if (row < n && l.g == 0) {
+    const T e = alpha * v[row] - beta * s;
+    out[row] = ADD ? out[row] + e : e;
+  }
 }
 
 // r = b - A x
-template <typename T>
+template <typename T, int G>
 __global__ __launch_bounds__(kBlock) void k_sell_resid(
   SellView A, const T* __restrict__ va, const T* __restrict__ x, const T* __restrict__ b,
   T* __restrict__ r, int n)
 {
-  const int row = blockIdx.x * blockDim.x + threadIdx.x;
-  if (row >= n) return;
-  r[row] = b[row] - sell_dot(A, va, x, row);
+  const SellLane l = sell_lane<G>();
+  if (l.row - l.row % (kWave / G) >= n) return;
+  const T s = sell_dot<T, G>(A, va, x, l);
+  if (l.row < n && l.g == 0) r[l.row] = b[l.row] - s;
 }
 
 // out[p] = T(a[slot[p]] * (colscale ? colscale[ci[p]] : 1)), 0 for padding
@@ -306,6 +322,24 @@ inline SellView sell_view(const Sell& s)
     default:                                                                 \
       kernel<T, 32, true><<<nw_blocks_, kBlock, 0, stream>>>(__VA_ARGS__);   \
     }                                                                        \
+  } while (0)
+
+// kernel<T, G> or kernel<T, G, true> of the sliced ELL kernels
+#define NW_SELL_LAUNCH(kernel, T, G, n, stream, ...)                         \
+  do {                                                                       \
+    const unsigned nw_blocks_ = grid_for((int64_t)(n) * (G), kBlock);        \
+    if ((G) == 1)                                                            \
+      kernel<T, 1><<<nw_blocks_, kBlock, 0, stream>>>(__VA_ARGS__);          \
+    else                                                                     \
+      kernel<T, 2><<<nw_blocks_, kBlock, 0, stream>>>(__VA_ARGS__);          \
+  } while (0)
+#define NW_SELL_LAUNCH_ADD(kernel, T, G, n, stream, ...)                     \
+  do {                                                                       \
+    const unsigned nw_blocks_ = grid_for((int64_t)(n) * (G), kBlock);        \
+    if ((G) == 1)                                                            \
+      kernel<T, 1, true><<<nw_blocks_, kBlock, 0, stream>>>(__VA_ARGS__);    \
+    else                                                                     \
+      kernel<T, 2, true><<<nw_blocks_, kBlock, 0, stream>>>(__VA_ARGS__);    \
   } while (0)
 
 #define NW_ROW_LAUNCH(kernel, T, G, n, stream, ...)                          \
