@@ -49,9 +49,12 @@ __global__ __launch_bounds__(kBlock) void k_mdot(MdotArgs a,
   const double om_interp = 1.0 - a.interp;
   double av[3];
   for (int d = 0; d < 3; ++d) av[d] = a.areav[3 * e + d];
-  const double udL = a.udiag[L], udR = a.udiag[R];
+  // the two ends' 1 / Udiag, once each (the formula divides by them eight
+  // times, fifteen instructions a division: 125 -> 111 us with them once each
+  // on a box of 5.8 M edges)
+  const double iudL = 1.0 / a.udiag[L], iudR = 1.0 / a.udiag[R];
   const double rhoL = a.rho[L], rhoR = a.rho[R];
-  const double projTimeScale = 0.5 * (1.0 / udL + 1.0 / udR);
+  const double projTimeScale = 0.5 * (iudL + iudR);
   const double rhoIp = 0.5 * (rhoL + rhoR);
   double dx[3], axdx = 0.0, asq = 0.0;
   for (int d = 0; d < 3; ++d) {
@@ -74,9 +77,9 @@ __global__ __launch_bounds__(kBlock) void k_mdot(MdotArgs a,
     const double uR = a.vel[3 * R + d], uL = a.vel[3 * L + d];
     const double rhoUjIp = 0.5 * (rhoR * uR + rhoL * uL);
     const double ujIp = 0.5 * (uR + uL);
-    double GjIp = 0.5 * (a.dpdx[3 * R + d] / udR + a.dpdx[3 * L + d] / udL);
+    double GjIp = 0.5 * (a.dpdx[3 * R + d] * iudR + a.dpdx[3 * L + d] * iudL);
     if constexpr (BUOY)
-      GjIp -= 0.5 * ((mR * a.src[3 * R + d]) / udR + (mL * a.src[3 * L + d]) / udL);
+      GjIp -= 0.5 * ((mR * a.src[3 * R + d]) * iudR + (mL * a.src[3 * L + d]) * iudL);
     tmdot += (a.interp * rhoUjIp + om_interp * rhoIp * ujIp + GjIp) * av[d] -
              kxj * GjIp * a.noc;
   }
