@@ -92,9 +92,10 @@ struct DevMat {
   const int32_t* dia_off = nullptr;  // level's slices
   const int32_t* base = nullptr;
   const uint16_t* cd = nullptr;
+  bool stretch = false;
   const T* v = nullptr;
   int64_t nv = 0;  // stored values (padding included)
-  SellView view() const { return {sp, ci, dia_w, dia_off, base, cd}; }
+  SellView view() const { return {sp, ci, dia_w, dia_off, base, cd, stretch}; }
   T* own_v = nullptr;  // v, but for the fine level (the solver's copy)
   Sell own;            // sliced ELL structure
   int32_t* own_rp = nullptr;
@@ -106,6 +107,12 @@ struct DevMat {
 // 1.5-1.9x over CSR, and the 20-24-entry operators of levels 1-2 cut the
 // whole solve by 5-10 %; the 36-200-entry coarser operators lose).
 constexpr double kSellMaxAvgRow = 25.0;
+// ... if there are this many rows: with fewer, a lane's walk over its row's
+// entries, eight at a time, is what bounds it (restrictions to 43.5 and 10.9
+// thousand rows of 15 and 13 entries, FP64: 21.3 and 18.1 us with two lanes;
+// in CSR 14.8 and 13.4 with 4 lanes, 9.2 and 8.2 with 8, 10.7 and 5.2 with
+// 16).  207 thousand rows of 12 entries take 12.6 us with two lanes.
+constexpr int64_t kSellMinRows = 200000;
 
 template <typename T>
 static void mat_spmv(const DevMat<T>& M, const T* x, T* y, T alpha,
@@ -412,11 +419,14 @@ static int device_lmax(int n, double* x, double* y, const double* dinv, const M&
 }
 
 // Uploads a host CSR matrix.  Rows of more than kSellMaxAvgRow entries on
-// average stay in CSR (G lanes per row); shorter ones are packed into sliced
-// ELL on the device from the uploaded CSR, with padding positions repeating
-// the row's last column (value 0), so that they stay inside the columns of
-// a rectangular P or R.
-static int upload_mat(const amg::Csr& h, DevMat<double>& d, hipStream_t st)
+// average, or fewer rows than kSellMinRows, stay in CSR: G lanes per row, that
+// take its average length at once, or four times that if the rows are ragged
+// (P and R: the longest has ten times the average; a level's own matrix is
+// slower with more lanes, 8.0 -> 10.3 us at twice as many for 43.5 thousand
+// rows of 28).  Others are packed into sliced ELL on the device from the
+// uploaded CSR, with padding positions repeating the row's last column (value
+// 0), so that they stay inside the columns of a rectangular P or R.
+static int upload_mat(const amg::Csr& h, DevMat<double>& d, bool ragged, hipStream_t st)
 {
   NW_REQUIRE(h.nrows >= 1 && h.nrows < INT32_MAX && h.ncols >= 1 && h.nnz() < INT32_MAX,
              NW_E_ARG, "AMG level too large or empty");
@@ -424,8 +434,8 @@ static int upload_mat(const amg::Csr& h, DevMat<double>& d, hipStream_t st)
   const double avg = (double)nnz / (double)n;
   const std::vector<int32_t> rp(h.rp.begin(), h.rp.end());
   d.n = (int)n;
-  if (avg > kSellMaxAvgRow) {
-    d.G = lanes_per_row(avg);
+  if (avg > kSellMaxAvgRow || n < kSellMinRows) {
+    d.G = lanes_per_row(ragged ? 4.0 * avg : avg);
     d.nv = nnz;
     NW_HIP(hipMalloc(&d.own_rp, sizeof(int32_t) * rp.size()));
     NW_HIP(hipMalloc(&d.own_ci, sizeof(int32_t) * std::max<int64_t>(nnz, 1)));
@@ -521,21 +531,22 @@ static int upload_hier(Ctx* c, const amg::Hierarchy& h, DevHier<double>& H)
       L.A.n = L.n;
       L.A.sp = c->g.sell.sp;
       L.A.ci = c->g.sell.ci;
+      L.A.stretch = sell_view(c->g.sell).stretch;
       L.A.dia_w = c->g.sell.dia_w;
       L.A.dia_off = c->g.sell.dia_off;
       L.A.base = c->g.sell.base;
       L.A.cd = c->g.sell.cd;
       L.A.nv = c->g.sell.len;
     } else {
-      int rc = upload_mat(hl.A, L.A, st);
+      int rc = upload_mat(hl.A, L.A, false, st);
       if (rc) return rc;
     }
     NW_HIP(hipMalloc(&L.dinv, sizeof(double) * std::max(L.n, 1)));
     NW_HIP(hipMemcpyAsync(L.dinv, hl.dinv.data(), sizeof(double) * L.n,
                           hipMemcpyHostToDevice, st));
     int rc = alloc_level_vectors(L);
-    if (!rc && l + 1 < nl) rc = upload_mat(hl.P, L.P, st);
-    if (!rc && l + 1 < nl) rc = upload_mat(hl.R, L.R, st);
+    if (!rc && l + 1 < nl) rc = upload_mat(hl.P, L.P, true, st);
+    if (!rc && l + 1 < nl) rc = upload_mat(hl.R, L.R, true, st);
     if (rc) return rc;
   }
   H.nc = (int)h.levels.back().A.nrows;
@@ -569,6 +580,7 @@ static int narrow_hier(Ctx* c, const DevHier<double>& D, DevHier<float>& H)
       L.A.n = S.A.n;
       L.A.sp = S.A.sp;
       L.A.ci = S.A.ci;
+      L.A.stretch = S.A.stretch;
       L.A.dia_w = S.A.dia_w;
       L.A.dia_off = S.A.dia_off;
       L.A.base = S.A.base;

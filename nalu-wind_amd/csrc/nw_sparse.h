@@ -16,17 +16,19 @@ constexpr int64_t kSellFillRows = 256 * 64 * 64;
 // Lanes per row for CSR rows of `avg` entries: each lane takes kCsrUnroll
 // entries per step as independent loads, so a row of average length is
 // covered by about one step (measured on the 20-entry AMG coarse operator
-// at 256^3: 8 lanes x 4 loads beat 16 lanes x 1 load by ~1.6x).
+// at 256^3: 8 lanes x 4 loads beat 16 lanes x 1 load by ~1.6x).  A whole wave
+// takes twice as many per step (4424 rows of 363 entries, FP32: 5.7 us, 9.1
+// with 32 lanes, four loads a step).
 constexpr int kCsrUnroll = 4;
 inline int lanes_per_row(double avg)
 {
   int g = 1;
-  while (g < 32 && g * kCsrUnroll < avg) g *= 2;
+  while (g < kWave && g * kCsrUnroll < avg) g *= 2;
   return g;
 }
 
 // Partial sum of row `row` over the entries g, g+G, ... (lane g of G),
-// kCsrUnroll entries per step loaded before any is used; padding entries
+// U = kCsrUnroll (G = 64: twice that) entries per step loaded before any is used; padding entries
 // repeat the row's last column with value 0.  Rows are contiguous, so the
 // G lanes of a row read consecutive entries.
 template <typename T, int G>
@@ -35,20 +37,21 @@ __device__ inline T csr_dot(const int32_t* __restrict__ rp,
                             const T* __restrict__ va, const T* __restrict__ x,
                             int row, int g)
 {
+  constexpr int U = G == kWave ? 2 * kCsrUnroll : kCsrUnroll;
   const int k0 = rp[row], k1 = rp[row + 1];
   T s = 0;
-  for (int k = k0 + g; k < k1; k += G * kCsrUnroll) {
-    int c[kCsrUnroll];
-    T v[kCsrUnroll];
+  for (int k = k0 + g; k < k1; k += G * U) {
+    int c[U];
+    T v[U];
 #pragma unroll
-    for (int u = 0; u < kCsrUnroll; ++u) {
+    for (int u = 0; u < U; ++u) {
       const int kk = k + u * G;
       const bool ok = kk < k1;
       c[u] = ci[ok ? kk : k1 - 1];
       v[u] = ok ? va[kk] : (T)0;
     }
 #pragma unroll
-    for (int u = 0; u < kCsrUnroll; ++u) s += v[u] * x[c[u]];
+    for (int u = 0; u < U; ++u) s += v[u] * x[c[u]];
   }
   return s;
 }
@@ -142,14 +145,27 @@ __global__ __launch_bounds__(kBlock) void k_resid(
 // offsets, which are the same for the whole wave (scalar loads with one
 // lane), and reads no column array; a slice in delta form (A.base[k] >= 0)
 // reads 16-bit columns relative to its base instead of the 32-bit columns.
+// The hardware deals workgroups to the 8 XCDs in turn.  With A.stretch
+// (matrices mostly in offset form: a box's, whose rows are alike) each XCD
+// takes one eighth of the rows instead, so that the x of a row's neighbours
+// is fetched into one L2 and not into several: 32.7 -> 25.1 us for the 4.2 M
+// 7-entry rows of a 160^3 box (FP32), 14.4 -> 12.5 for 0.96 M (FP64).  Coarse
+// AMG levels' rows are longer in one part of a stretched mesh than in
+// another: the XCDs' shares differ (27 -> 39 us on the 933 thousand rows of
+// its level 1), and stretches of 1 to 16 thousand rows gain nothing.
 struct SellLane {
   int row, g;
 };
 template <int G>
-__device__ inline SellLane sell_lane()
+__device__ inline SellLane sell_lane(bool stretch)
 {
   constexpr int R = kWave / G;
-  const int t = blockIdx.x * kBlock + threadIdx.x;
+  unsigned b = blockIdx.x;
+  if (stretch) {
+    const unsigned q = gridDim.x / 8, r = gridDim.x % 8, xcd = b % 8;
+    b = xcd * q + min(xcd, r) + b / 8;
+  }
+  const int t = b * kBlock + threadIdx.x;
   const int lane = t & (kWave - 1);
   return {(t / kWave) * R + lane % R, lane / R};
 }
@@ -207,7 +223,7 @@ __global__ __launch_bounds__(kBlock) void k_sell_spmv(
   SellView A, const T* __restrict__ va, const T* __restrict__ x, T* __restrict__ y, int n,
   T alpha)
 {
-  const SellLane l = sell_lane<G>();
+  const SellLane l = sell_lane<G>(A.stretch);
   if (l.row - l.row % (kWave / G) >= n) return;  // whole waves
   const T s = sell_dot<T, G>(A, va, x, l);
   if (l.row < n && l.g == 0) y[l.row] = alpha * s;
@@ -218,7 +234,7 @@ template <typename T, int G>
 __global__ __launch_bounds__(kBlock) void k_sell_spmv_add(
   SellView A, const T* __restrict__ va, const T* __restrict__ x, T* __restrict__ y, int n)
 {
-  const SellLane l = sell_lane<G>();
+  const SellLane l = sell_lane<G>(A.stretch);
   if (l.row - l.row % (kWave / G) >= n) return;
   const T s = sell_dot<T, G>(A, va, x, l);
   if (l.row < n && l.g == 0) y[l.row] += s;
@@ -231,7 +247,7 @@ __global__ __launch_bounds__(kBlock) void k_sell_cheb_step(
   const T* __restrict__ dinv, T* __restrict__ d, T* __restrict__ zo, int n,
   T c1, T c2)
 {
-  const SellLane l = sell_lane<1>();
+  const SellLane l = sell_lane<1>(A.stretch);
   const int row = l.row;
   if (row >= n) return;
   const T s = sell_dot<T, 1>(A, va, z, l);
@@ -246,7 +262,7 @@ __global__ __launch_bounds__(kBlock) void k_sell_smooth(
   SellView A, const T* __restrict__ va, const T* __restrict__ v, T* __restrict__ out, int n,
   T alpha, T beta)
 {
-  const SellLane l = sell_lane<G>();
+  const SellLane l = sell_lane<G>(A.stretch);
   const int row = l.row;
   if (row - row % (kWave / G) >= n) return;
   const T s = sell_dot<T, G>(A, va, v, l);
@@ -262,7 +278,7 @@ __global__ __launch_bounds__(kBlock) void k_sell_resid(
   SellView A, const T* __restrict__ va, const T* __restrict__ x, const T* __restrict__ b,
   T* __restrict__ r, int n)
 {
-  const SellLane l = sell_lane<G>();
+  const SellLane l = sell_lane<G>(A.stretch);
   if (l.row - l.row % (kWave / G) >= n) return;
   const T s = sell_dot<T, G>(A, va, x, l);
   if (l.row < n && l.g == 0) r[l.row] = b[l.row] - s;
@@ -295,7 +311,7 @@ void sell_free(Sell& s);
 
 inline SellView sell_view(const Sell& s)
 {
-  return {s.sp, s.ci, s.dia_w, s.dia_off, s.base, s.cd};
+  return {s.sp, s.ci, s.dia_w, s.dia_off, s.base, s.cd, 2 * s.dia_slices > s.nslices};
 }
 
 // launch helper: dispatch a G-templated row kernel by lanes-per-row
@@ -319,8 +335,11 @@ inline SellView sell_view(const Sell& s)
     case 16:                                                                 \
       kernel<T, 16, true><<<nw_blocks_, kBlock, 0, stream>>>(__VA_ARGS__);   \
       break;                                                                 \
-    default:                                                                 \
+    case 32:                                                                 \
       kernel<T, 32, true><<<nw_blocks_, kBlock, 0, stream>>>(__VA_ARGS__);   \
+      break;                                                                 \
+    default:                                                                 \
+      kernel<T, 64, true><<<nw_blocks_, kBlock, 0, stream>>>(__VA_ARGS__);   \
     }                                                                        \
   } while (0)
 
@@ -361,8 +380,11 @@ inline SellView sell_view(const Sell& s)
     case 16:                                                                 \
       kernel<T, 16><<<nw_blocks_, kBlock, 0, stream>>>(__VA_ARGS__);         \
       break;                                                                 \
-    default:                                                                 \
+    case 32:                                                                 \
       kernel<T, 32><<<nw_blocks_, kBlock, 0, stream>>>(__VA_ARGS__);         \
+      break;                                                                 \
+    default:                                                                 \
+      kernel<T, 64><<<nw_blocks_, kBlock, 0, stream>>>(__VA_ARGS__);         \
     }                                                                        \
   } while (0)
 

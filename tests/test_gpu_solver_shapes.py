@@ -102,3 +102,20 @@ def test_amg_levels(nw, ctx, shape, mode):
     B.apply_dirichlet(top, 0, 1, P.p, np.zeros(P.n))
     r = B.rhs - B.spmv(ctx.solution())
     assert s2.converged and np.linalg.norm(r) <= 1.0001 * tol * np.linalg.norm(B.rhs)
+
+
+@pytest.mark.parametrize("mode", [0, 1])
+def test_amg_levels_of_every_layout(nw, ctx, mode):
+    """Large enough for sliced ELL and wide CSR levels: two lanes per row; a
+    wave per row (a restriction of more than 32 entries a row, two or more for
+    each row of the finer level); a row count that the 8 dies do not share
+    evenly."""
+    P, A = _system(nw, ctx, (97, 95, 101))
+    tol = 1e-8
+    st = ctx.solve(nw.solver_cfg(kspace=30, max_iters=300, tol=tol, precond=nw.PREC_AMG,
+                                 mode=mode, inner_tol=1e-4))
+    levels = [tuple(l)[:2] for l in ctx.amg_levels()]
+    assert any(200000 <= n < 1000000 and 8 * n <= nnz <= 25 * n for n, nnz in levels[1:-1]), levels
+    assert any(f > 16 * c for (f, _), (c, _) in zip(levels[1:], levels[2:])), levels
+    r = A.rhs - A.spmv(ctx.solution())
+    assert st.converged and np.linalg.norm(r) <= 1.0001 * tol * np.linalg.norm(A.rhs)
