@@ -122,7 +122,7 @@ struct SellView {
   const int32_t* dia_off;
   const int32_t* base;     // null: no slice in delta form
   const uint16_t* cd;
-  bool stretch;            // an XCD takes one stretch of the rows (row_block)
+  bool stretch;            // an XCD takes stretches of the rows (sell_lane)
 };
 
 struct Graph {

@@ -147,12 +147,16 @@ __global__ __launch_bounds__(kBlock) void k_resid(
 // reads 16-bit columns relative to its base instead of the 32-bit columns.
 // The hardware deals workgroups to the 8 XCDs in turn.  With A.stretch
 // (matrices mostly in offset form: a box's, whose rows are alike) each XCD
-// takes one eighth of the rows instead, so that the x of a row's neighbours
-// is fetched into one L2 and not into several: 32.7 -> 25.1 us for the 4.2 M
-// 7-entry rows of a 160^3 box (FP32), 14.4 -> 12.5 for 0.96 M (FP64).  Coarse
-// AMG levels' rows are longer in one part of a stretched mesh than in
-// another: the XCDs' shares differ (27 -> 39 us on the 933 thousand rows of
-// its level 1), and stretches of 1 to 16 thousand rows gain nothing.
+// takes stretches of kStretch blocks (131 thousand rows) instead, so that the
+// x of a row's neighbours is fetched into one L2 and not into several:
+// 32.7 -> 25.7 us for the 4.2 M 7-entry rows of a 160^3 box (FP32), 14.4 ->
+// 12.5 for 0.96 M (FP64), 251 -> 238 for 17 M (FP64).  One eighth of the rows
+// to each is slower on large boxes (17 M rows, FP64: 256), 2048 blocks too
+// (245).  Coarse AMG levels' rows are longer in one part of a stretched mesh
+// than in another: the XCDs' shares differ (27 -> 39 us on the 933 thousand
+// rows of a 160^3 box's level 1), and stretches of 1 to 16 thousand rows gain
+// nothing.
+constexpr unsigned kStretch = 512;
 struct SellLane {
   int row, g;
 };
@@ -162,8 +166,10 @@ __device__ inline SellLane sell_lane(bool stretch)
   constexpr int R = kWave / G;
   unsigned b = blockIdx.x;
   if (stretch) {
-    const unsigned q = gridDim.x / 8, r = gridDim.x % 8, xcd = b % 8;
-    b = xcd * q + min(xcd, r) + b / 8;
+    const unsigned first = b / (8 * kStretch) * (8 * kStretch);  // of its round
+    const unsigned size = min(8 * kStretch, gridDim.x - first);
+    const unsigned q = size / 8, r = size % 8, xcd = b % 8;
+    b = first + xcd * q + min(xcd, r) + (b - first) / 8;
   }
   const int t = b * kBlock + threadIdx.x;
   const int lane = t & (kWave - 1);

@@ -104,13 +104,14 @@ def test_amg_levels(nw, ctx, shape, mode):
     assert s2.converged and np.linalg.norm(r) <= 1.0001 * tol * np.linalg.norm(B.rhs)
 
 
-@pytest.mark.parametrize("mode", [0, 1])
-def test_amg_levels_of_every_layout(nw, ctx, mode):
+@pytest.mark.parametrize("mode, shape", [(0, (97, 95, 101)), (1, (97, 95, 101)),
+                                         (0, (104, 103, 102))])
+def test_amg_levels_of_every_layout(nw, ctx, mode, shape):
     """Large enough for sliced ELL and wide CSR levels: two lanes per row; a
     wave per row (a restriction of more than 32 entries a row, two or more for
     each row of the finer level); a row count that the 8 dies do not share
-    evenly."""
-    P, A = _system(nw, ctx, (97, 95, 101))
+    evenly, within one round of their stretches (8 x 131072 rows) and past it."""
+    P, A = _system(nw, ctx, shape)
     tol = 1e-8
     st = ctx.solve(nw.solver_cfg(kspace=30, max_iters=300, tol=tol, precond=nw.PREC_AMG,
                                  mode=mode, inner_tol=1e-4))
