@@ -7,6 +7,7 @@
 #pragma once
 
 #include "nw_internal.h"
+#include "nw_sell.h"
 
 namespace nw {
 
@@ -142,8 +143,8 @@ __global__ __launch_bounds__(kBlock) void k_resid(
 // reads x at a valid column with value 0.  With one lane the row sum runs
 // over j in order; G lanes' sums are added by a fixed butterfly.  A slice in
 // offset form (A.dia_w[k] > 0) takes its columns as row + the slice's
-// offsets, which are the same for the whole wave (scalar loads with one
-// lane), and reads no column array; a slice in delta form (A.base[k] >= 0)
+// offsets (dia_column), which are the same for the whole wave (scalar loads
+// with one lane), and reads no column array; a slice in delta form (A.base[k] >= 0)
 // reads 16-bit columns relative to its base instead of the 32-bit columns.
 // The hardware deals workgroups to the 8 XCDs in turn.  With A.stretch
 // (matrices mostly in offset form: a box's, whose rows are alike) each XCD
@@ -178,7 +179,7 @@ __device__ inline SellLane sell_lane(bool stretch)
 
 template <typename T, int G>
 __device__ inline T sell_dot(const SellView& A, const T* __restrict__ va,
-                             const T* __restrict__ x, SellLane l)
+                             const T* __restrict__ x, SellLane l, int n)
 {
   // rows of one wave are in one slice: the slice index is wave-uniform
   const int row = l.row;
@@ -203,7 +204,7 @@ __device__ inline T sell_dot(const SellView& A, const T* __restrict__ va,
   const int base = A.base ? A.base[k] : -1;
   if (A.dia_w && A.dia_w[k] > 0) {
     const int32_t* off = A.dia_off + (int64_t)k * kDiaMax;
-    sum([&](int j) { return row + off[j]; });
+    sum([&](int j) { return dia_column(row, off[j], n); });
   } else if (base >= 0) {
     sum([&](int j) { return base + A.cd[b + 64 * (int64_t)j]; });
   } else {
@@ -231,7 +232,7 @@ __global__ __launch_bounds__(kBlock) void k_sell_spmv(
 {
   const SellLane l = sell_lane<G>(A.stretch);
   if (l.row - l.row % (kWave / G) >= n) return;  // whole waves
-  const T s = sell_dot<T, G>(A, va, x, l);
+  const T s = sell_dot<T, G>(A, va, x, l, n);
   if (l.row < n && l.g == 0) y[l.row] = alpha * s;
 }
 
@@ -242,7 +243,7 @@ __global__ __launch_bounds__(kBlock) void k_sell_spmv_add(
 {
   const SellLane l = sell_lane<G>(A.stretch);
   if (l.row - l.row % (kWave / G) >= n) return;
-  const T s = sell_dot<T, G>(A, va, x, l);
+  const T s = sell_dot<T, G>(A, va, x, l, n);
   if (l.row < n && l.g == 0) y[l.row] += s;
 }
 
@@ -256,7 +257,7 @@ __global__ __launch_bounds__(kBlock) void k_sell_cheb_step(
   const SellLane l = sell_lane<1>(A.stretch);
   const int row = l.row;
   if (row >= n) return;
-  const T s = sell_dot<T, 1>(A, va, z, l);
+  const T s = sell_dot<T, 1>(A, va, z, l, n);
   const T dn = c1 * d[row] + c2 * dinv[row] * (v[row] - s);
   d[row] = dn;
   zo[row] = z[row] + dn;
@@ -271,7 +272,7 @@ __global__ __launch_bounds__(kBlock) void k_sell_smooth(
   const SellLane l = sell_lane<G>(A.stretch);
   const int row = l.row;
   if (row - row % (kWave / G) >= n) return;
-  const T s = sell_dot<T, G>(A, va, v, l);
+  const T s = sell_dot<T, G>(A, va, v, l, n);
   if (row < n && l.g == 0) {
     const T e = alpha * v[row] - beta * s;
     out[row] = ADD ? out[row] + e : e;
@@ -286,7 +287,7 @@ __global__ __launch_bounds__(kBlock) void k_sell_resid(
 {
   const SellLane l = sell_lane<G>(A.stretch);
   if (l.row - l.row % (kWave / G) >= n) return;
-  const T s = sell_dot<T, G>(A, va, x, l);
+  const T s = sell_dot<T, G>(A, va, x, l, n);
   if (l.row < n && l.g == 0) r[l.row] = b[l.row] - s;
 }
 

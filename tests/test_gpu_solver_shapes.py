@@ -120,3 +120,19 @@ def test_amg_levels_of_every_layout(nw, ctx, mode, shape):
     assert any(f > 16 * c for (f, _), (c, _) in zip(levels[1:], levels[2:])), levels
     r = A.rhs - A.spmv(ctx.solution())
     assert st.converged and np.linalg.norm(r) <= 1.0001 * tol * np.linalg.norm(A.rhs)
+
+
+@pytest.mark.parametrize("mode,prec", [(0, 3), (1, 3), (0, 1), (1, 2)])
+def test_last_slice_of_one_row(nw, ctx, mode, prec):
+    """65^3 nodes: the fine matrix in offset form up to a last slice of a
+    single row, whose 63 other lanes read the row's own columns."""
+    P, A = _system(nw, ctx, (64, 64, 64))
+    assert P.n % 64 == 1
+    tol = 1e-8
+    st = ctx.solve(nw.solver_cfg(kspace=50, max_iters=400, tol=tol, precond=prec, mode=mode,
+                                 inner_tol=1e-4, cheb_degree=4, cheb_ratio=30.0),
+                   raise_on_noconv=False)
+    x = ctx.solution()
+    rel = np.linalg.norm(A.rhs - A.spmv(x)) / np.linalg.norm(A.rhs)
+    assert st.final_rel == pytest.approx(rel, rel=1e-3)
+    assert rel <= 1.0001 * tol if prec == 3 else rel < 0.1
