@@ -1234,7 +1234,23 @@ int nw_linsys_solve(nw_ctx* c, const nw_solver_cfg* cfg, nw_solve_stats* out)
   if (cheb && !k->pe) NW_HIP(hipMalloc(&k->pe, sizeof(double) * 2 * n));
 
   hipStream_t st = c->stream;
+  // k->dinv = 1 / diag; refuses a zero or non-finite diagonal
+  auto diag_inv = [&]() -> int {
+    NW_HIP(hipMemsetAsync(k->bad, 0, sizeof(int), st));
+    k_diag_inv<<<grid_for(n, kBlock), kBlock, 0, st>>>(c->g.diag, c->g.vals,
+                                                      k->dinv, (int)n, k->bad);
+    NW_LAUNCH_CHECK();
+    int bad = 0;
+    NW_HIP(hipMemcpyAsync(&bad, k->bad, sizeof(int), hipMemcpyDeviceToHost, st));
+    NW_HIP(hipStreamSynchronize(st));
+    NW_REQUIRE(!bad, NW_E_NONFINITE, "zero or non-finite diagonal in the matrix");
+    return NW_OK;
+  };
   if (amgp && (!c->amg || !cfg->reuse_preconditioner)) {
+    // before the setup: a hierarchy outlives this call, and its 1 / diag (0
+    // for a zero diagonal) scales the operator of every solve that reuses it
+    rc = diag_inv();
+    if (rc) return rc;
     amg_free(c->amg);
     c->amg = nullptr;
     rc = amg_setup(c, &c->amg);
@@ -1254,14 +1270,8 @@ int nw_linsys_solve(nw_ctx* c, const nw_solver_cfg* cfg, nw_solve_stats* out)
   Solve S{c, k, cfg, lanes_per_row((double)nnz / std::max<int64_t>(n, 1))};
   S.st = st;
   // preconditioner setup: 1/diag, the matrix in the cycle type
-  NW_HIP(hipMemsetAsync(k->bad, 0, sizeof(int), st));
-  k_diag_inv<<<grid_for(n, kBlock), kBlock, 0, st>>>(c->g.diag, c->g.vals,
-                                                    k->dinv, (int)n, k->bad);
-  NW_LAUNCH_CHECK();
-  int bad = 0;
-  NW_HIP(hipMemcpyAsync(&bad, k->bad, sizeof(int), hipMemcpyDeviceToHost, st));
-  NW_HIP(hipStreamSynchronize(st));
-  NW_REQUIRE(!bad, NW_E_NONFINITE, "zero or non-finite diagonal in the matrix");
+  rc = diag_inv();
+  if (rc) return rc;
   const double* colscale = cfg->precond == NW_PREC_JACOBI ? k->dinv
                            : amgp                         ? amg_fine_dinv(c->amg)
                                                           : nullptr;

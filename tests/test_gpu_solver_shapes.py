@@ -136,3 +136,23 @@ def test_last_slice_of_one_row(nw, ctx, mode, prec):
     rel = np.linalg.norm(A.rhs - A.spmv(x)) / np.linalg.norm(A.rhs)
     assert st.final_rel == pytest.approx(rel, rel=1e-3)
     assert rel <= 1.0001 * tol if prec == 3 else rel < 0.1
+
+
+@pytest.mark.parametrize("mode", [0, 1])
+def test_refused_matrix_leaves_no_hierarchy(nw, ctx, mode):
+    """An AMG solve that a zero diagonal ends, then one on the good matrix
+    with reuse on: its hierarchy must be of that matrix, whose columns it
+    scales."""
+    P, A = _system(nw, ctx, (12, 11, 10))
+    cfg = nw.solver_cfg(kspace=30, max_iters=200, tol=1e-8, precond=nw.PREC_AMG, mode=mode,
+                        inner_tol=1e-4, reuse_preconditioner=1)
+    ctx.reset_rows([P.n // 2], 0, 1, diag=0.0)
+    with pytest.raises(nw.NwError) as ei:
+        ctx.solve(cfg)
+    assert ei.value.code == nw.E_NONFINITE
+    ctx.assemble_continuity(nw.continuity_defaults())  # the same graph
+    top = np.where(np.abs(P.coords[:, 2] - 1.0) < 1e-12)[0].astype(np.int32)
+    ctx.apply_dirichlet(top, nw.F_PRESSURE, nw.F_DIFF_FLUX_COEFF, 0, 1)
+    st = ctx.solve(cfg)
+    r = A.rhs - A.spmv(ctx.solution())
+    assert st.converged and np.linalg.norm(r) <= 1.0001e-8 * np.linalg.norm(A.rhs)
