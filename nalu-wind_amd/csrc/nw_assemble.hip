@@ -74,6 +74,16 @@ __device__ inline double van_leer(double dqm, double dqp, double eps)
   return (2.0 * (p + fabs(p))) / ((dqm + dqp) * (dqm + dqp) + eps);
 }
 
+// 0.5 (a b + c d) with (a, b) and (c, d) interchangeable.  No contraction: of
+// fma(a, b, c d) and fma(c, d, a b) the two ends of an edge, which each see
+// the other as the second, would take one each, and the flux out of one would
+// not be the flux into the other.
+__device__ inline double mean_product(double a, double b, double c, double d)
+{
+#pragma clang fp contract(off)
+  return 0.5 * (a * b + c * d);
+}
+
 // ------------------------------------------------------------------ physics
 // Each physics type has a Node record of the fields one node contributes,
 // load(n, rec), derive(rec) (quantities of the node alone, formed once per
@@ -85,7 +95,8 @@ __device__ inline double van_leer(double dqm, double dqp, double eps)
 // area vector and the mass flow rate taken out of that end: swapping the ends
 // changes the sign of A, dx, mdot and the fluxes and exchanges the rows.
 // orient(er, side) turns the edge's values out of node[side], so one body
-// serves both ends and the lanes of a wave need not agree on the side.
+// serves both ends and the lanes of a wave need not agree on the side.  Every
+// expression gives the same value, or exactly its negative, from either end.
 //
 // FP64 divisions (about fifteen instructions each) are kept to those that the
 // formulas need per edge: uniform divisors (relaxation, time scale) come as
@@ -143,9 +154,11 @@ struct ContinuityPhysT {
     }
   }
 
-  // ud becomes 1 / Udiag, g and s the terms they divide
+  // ud becomes 1 / Udiag, g and s the terms they divide; rounded here, not
+  // fused into the two ends' sum (mean_product)
   __device__ void derive(Node& r) const
   {
+#pragma clang fp contract(off)
     r.ud = 1.0 / r.ud;
     for (int d = 0; d < 3; ++d) {
       r.g[d] *= r.ud;
@@ -196,7 +209,7 @@ struct ContinuityPhysT {
     }
     for (int d = 0; d < 3; ++d) {
       const double kxj = av[d] - asq * inv_axdx * dx[d];
-      const double rhoUjIp = 0.5 * (R.rho * R.u[d] + L.rho * L.u[d]);
+      const double rhoUjIp = mean_product(R.rho, R.u[d], L.rho, L.u[d]);
       const double ujIp = 0.5 * (R.u[d] + L.u[d]);
       double GjIp = 0.5 * (R.g[d] + L.g[d]);
       if constexpr (BUOY) GjIp -= 0.5 * (R.s[d] + L.s[d]);

@@ -127,3 +127,39 @@ def test_zero_length_edge(nw, ctx):
     ctx.set_check_finite(True)
     with pytest.raises(nw.NwError, match="non-finite"):
         ctx.assemble_continuity(o)
+
+
+def test_what_leaves_one_end_of_an_edge_enters_the_other(nw, ctx):
+    """Edges that share no node: a row's right-hand side is one flux, and the
+    two ends' must be each other's negatives to the last bit, whichever end
+    the kernel looks from (a closed mesh loses nothing)."""
+    rng = np.random.default_rng(11)
+    ne = 3000
+    coords = rng.normal(size=(2 * ne, 3))
+    perm = rng.permutation(2 * ne).astype(np.int32).reshape(ne, 2)
+    edges = np.sort(perm, axis=1)
+    L, R = edges[:, 0], edges[:, 1]
+    areav = (coords[R] - coords[L]) * rng.uniform(0.5, 1.5, (ne, 1)) + rng.normal(size=(ne, 3)) * 0.2
+    P = pb.Problem.from_graph(coords, edges, areav, seed=3)
+
+    def opposite(ndof):
+        rhs = ctx.download()[3].reshape(-1, ndof)
+        assert np.count_nonzero(rhs[L]) > 0.9 * rhs[L].size
+        np.testing.assert_array_equal(rhs[L], -rhs[R])
+
+    P.upload(ctx)
+    ctx.build_graph(1)
+    for kw in ({}, {"interp_together": 0.0}, {"incompressible": 1.0}):
+        ctx.assemble_continuity(nw.continuity_defaults(**kw))
+        opposite(1)
+    for limiter in (0, 1):
+        s = nw.scalar_defaults(use_limiter=limiter, peclet=nw.Peclet(limiter, 1.0, 2.0, 4.0))
+        ctx.assemble_scalar(s)
+        opposite(1)
+    ctx.build_graph(3)
+    for limiter in (0, 1):
+        m = nw.momentum_defaults(alpha=0.5, use_limiter=limiter)
+        ctx.assemble_momentum(m)
+        opposite(3)
+        ctx.assemble_momentum_with_peclet(m, nw.Peclet(limiter, 1.0, 2.0, 4.0))
+        opposite(3)
