@@ -1116,7 +1116,7 @@ struct Mpnn {
   float* dPT = nullptr;    // W_in^T (the input layers read it k-major)
   float* w = nullptr;      // [nnz] slot weights
   std::vector<float*> h;   // L+1 activations [n][H]
-  std::vector<float*> msg; // messages m_l [n][H] (L when training, else 1)
+  std::vector<float*> msg; // messages m_l [n][H] (L when training, else 0)
   float *gs = nullptr, *gz = nullptr;
   float *feat = nullptr, *target = nullptr, *delta = nullptr, *dd = nullptr;
   double* r = nullptr;     // FP64 residual of x0
@@ -1246,42 +1246,40 @@ int check_graph(Mpnn* m)
   return NW_OK;
 }
 
+// Allocates what is missing of `count` activation arrays [n][H] of v.
+int ensure_rows(Mpnn* m, std::vector<float*>& v, int count)
+{
+  while ((int)v.size() < count) {
+    float* p = nullptr;
+    NW_HIP(hipMalloc(&p, sizeof(float) * m->n * m->H));
+    v.push_back(p);
+  }
+  return NW_OK;
+}
+
+// What every prediction and training sample needs, and with `training` the
+// activations, messages and gradients of all layers (the FP32 and bfloat16
+// predictions allocate their two activation arrays on first use).
 int ensure_buffers(Mpnn* m, bool training)
 {
   const int64_t n = m->n;
-  if (!m->w) {
-    NW_HIP(hipMalloc(&m->w, sizeof(float) * m->nnz));
-    NW_HIP(hipMalloc(&m->feat, sizeof(float) * kF * n));
-    NW_HIP(hipMalloc(&m->target, sizeof(float) * n));
-    NW_HIP(hipMalloc(&m->delta, sizeof(float) * n));
-    NW_HIP(hipMalloc(&m->dd, sizeof(float) * 2 * n));
-    NW_HIP(hipMalloc(&m->r, sizeof(double) * n));
-    NW_HIP(hipMalloc(&m->xb, sizeof(double) * n));
+  if (!m->w) NW_HIP(hipMalloc(&m->w, sizeof(float) * m->nnz));
+  if (!m->feat) NW_HIP(hipMalloc(&m->feat, sizeof(float) * kF * n));
+  if (!m->target) NW_HIP(hipMalloc(&m->target, sizeof(float) * n));
+  if (!m->delta) NW_HIP(hipMalloc(&m->delta, sizeof(float) * n));
+  if (!m->dd) NW_HIP(hipMalloc(&m->dd, sizeof(float) * 2 * n));
+  if (!m->r) NW_HIP(hipMalloc(&m->r, sizeof(double) * n));
+  if (!m->xb) NW_HIP(hipMalloc(&m->xb, sizeof(double) * n));
+  if (!m->partial)
     NW_HIP(hipMalloc(&m->partial, sizeof(double) * (size_t)kGradBlocks * m->nv));
-    NW_HIP(hipMalloc(&m->red, sizeof(double) * m->nv));
-    m->h.assign(2, nullptr);
-    for (auto& p : m->h) NW_HIP(hipMalloc(&p, sizeof(float) * n * m->H));
-    m->msg.assign(1, nullptr);
-    NW_HIP(hipMalloc(&m->msg[0], sizeof(float) * n * m->H));
-  }
-  if (training && (int)m->msg.size() < m->L) {
-    while ((int)m->msg.size() < m->L) {
-      float* p = nullptr;
-      NW_HIP(hipMalloc(&p, sizeof(float) * n * m->H));
-      m->msg.push_back(p);
-    }
-  }
-  if (training && (int)m->h.size() < m->L + 1) {
-    while ((int)m->h.size() < m->L + 1) {
-      float* p = nullptr;
-      NW_HIP(hipMalloc(&p, sizeof(float) * n * m->H));
-      m->h.push_back(p);
-    }
-  }
+  if (!m->red) NW_HIP(hipMalloc(&m->red, sizeof(double) * m->nv));
   if (!m->vd) NW_HIP(hipMalloc(&m->vd, sizeof(float) * n));
-  if (training && !m->gs) {
-    NW_HIP(hipMalloc(&m->gs, sizeof(float) * n * m->H));
-    NW_HIP(hipMalloc(&m->gz, sizeof(float) * n * m->H));
+  if (training) {
+    int rc = ensure_rows(m, m->h, m->L + 1);
+    if (!rc) rc = ensure_rows(m, m->msg, m->L);
+    if (rc) return rc;
+    if (!m->gs) NW_HIP(hipMalloc(&m->gs, sizeof(float) * n * m->H));
+    if (!m->gz) NW_HIP(hipMalloc(&m->gz, sizeof(float) * n * m->H));
   }
   return NW_OK;
 }
@@ -1379,6 +1377,8 @@ int forward_h(Mpnn* m, const float* feat, bool keep)
   hipStream_t st = c->stream;
   const Off o(H, L);
   const float* WT = m->dPT;
+  const int rc = ensure_rows(m, m->h, 2);
+  if (rc) return rc;
   k_input_layer<H><<<grid_for((int64_t)n * (H / 4), kBlock), kBlock, 0, st>>>(
     feat, WT, m->dP + o.bin, m->h[0], n);
   NW_LAUNCH_CHECK();
@@ -1721,6 +1721,9 @@ int nw_mpnn_record(nw_mpnn* m)
              "no solve has run on this system yet (nothing to record)");
   NW_HIP(hipSetDevice(m->c->device));
   rc = ensure_buffers(m, false);
+  // of the arrays that training on the sample takes
+  if (!rc) rc = ensure_rows(m, m->h, 2);
+  if (!rc) rc = ensure_rows(m, m->msg, 1);
   if (rc) return rc;
   Sample s;
   if (hipMalloc(&s.feat, sizeof(float) * kF * m->n) != hipSuccess ||

@@ -2,6 +2,8 @@
 tile of 16, partial tiles, fewer tiles than the eight stretches of the grid,
 rows of more than the eight slots a tile loads ahead (mixed meshes), both
 widths and several depths."""
+import ctypes
+
 import numpy as np
 import pytest
 
@@ -69,3 +71,35 @@ def test_layers_match_oracle(nw, ctx, mesh, H, L):
     d = orc.mpnn_forward(p, H, L, A, w, f2)
     np.testing.assert_allclose((x[inner] - xb[inner]) / so, d[inner], rtol=0,
                                atol=2e-5 * np.abs(d).max() + 4e-16 * np.abs(xb).max() / so)
+
+
+@pytest.mark.parametrize("precision,arrays", [("MPNN_BF16", 1.0), ("MPNN_FP32", 2.0)])
+def test_prediction_holds_its_own_activations_only(nw, ctx, precision, arrays):
+    """Device memory that a first prediction takes: two activation arrays of
+    its precision (in units of one FP32 array [n][H]), the small per-node and
+    per-slot arrays and the gradient partials; half an array more is within
+    the allocator's granularity, a message array or the other precision's
+    activations are not."""
+    def free_memory():  # of the runtime that the library is linked to
+        free, total = ctypes.c_size_t(), ctypes.c_size_t()
+        assert nw.lib.hipMemGetInfo(ctypes.byref(free), ctypes.byref(total)) == 0
+        return free.value
+
+    P = pb.Problem(64, 64, 64, seed=2)
+    P.upload(ctx)
+    ctx.build_graph(1)
+    ctx.assemble_continuity(nw.continuity_defaults())
+    ctx.set_solution(np.random.default_rng(1).normal(size=P.n))
+    ctx.solve(nw.solver_cfg(kspace=1, max_iters=0, x0=nw.X0_SOLUTION), raise_on_noconv=False)
+    H, L = 64, 1
+    net = nw.Mpnn(ctx, H, L, seed=3)
+    net.params = 0.1 * np.random.default_rng(2).normal(size=net.nparams)
+    net.precision = getattr(nw, precision)
+    free = free_memory()
+    net.predict()
+    used = free - free_memory()
+    row = 4 * P.n * H
+    nnz = P.n + 2 * P.ne
+    partials = 8 * 512 * (2 * H + 2 + L * H * (2 * H + 1) + 6 * H + 1)
+    small = 4 * nnz + 4 * P.n * (5 + 5) + 8 * P.n * 3
+    assert used < (arrays + 0.5) * row + partials + small
