@@ -975,6 +975,8 @@ struct Solve {
         *kdim = (int)(v & 0xff);
         return NW_OK;
       }
+      __builtin_ia32_pause();  // a whole AMG step goes by here: leave the core's
+                               // other thread and the memory bus alone
       if (spin % 4096 == 0) {
         const hipError_t e = hipStreamQuery(st);
         if (e == hipErrorNotReady) {
