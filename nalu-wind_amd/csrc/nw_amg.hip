@@ -111,8 +111,12 @@ constexpr double kSellMaxAvgRow = 25.0;
 // entries, eight at a time, is what bounds it (restrictions to 43.5 and 10.9
 // thousand rows of 15 and 13 entries, FP64: 21.3 and 18.1 us with two lanes;
 // in CSR 14.8 and 13.4 with 4 lanes, 9.2 and 8.2 with 8, 10.7 and 5.2 with
-// 16).  207 thousand rows of 12 entries take 12.6 us with two lanes.
-constexpr int64_t kSellMinRows = 200000;
+// 16).  The line by whole iterations of graded boxes, FP64, level 1 (rows of
+// 20 entries, its restriction and the level's own matrix) in sliced ELL / in
+// CSR: 48 thousand rows 172 / 167 us, 59 182 / 179, 67 187.5 / 186, 77 191 /
+// 194.5, 90 204 / 209, 114 231 / 240, 132 248 / 262, 161 279 / 295, 189 306 /
+// 328; FP32 from equal at 77 to 215 / 232 at 161.
+constexpr int64_t kSellMinRows = 70000;
 
 template <typename T>
 static void mat_spmv(const DevMat<T>& M, const T* x, T* y, T alpha,

@@ -156,3 +156,18 @@ def test_refused_matrix_leaves_no_hierarchy(nw, ctx, mode):
     st = ctx.solve(cfg)
     r = A.rhs - A.spmv(ctx.solution())
     assert st.converged and np.linalg.norm(r) <= 1.0001e-8 * np.linalg.norm(A.rhs)
+
+
+@pytest.mark.parametrize("mode", [0, 1])
+@pytest.mark.parametrize("shape,sliced", [((67, 66, 65), False), ((76, 75, 74), True)])
+def test_amg_levels_about_the_sliced_ell_line(nw, ctx, mode, shape, sliced):
+    """A level on either side of the 70 thousand rows from which levels are in
+    sliced ELL form, two lanes per row."""
+    P, A = _system(nw, ctx, shape)
+    tol = 1e-8
+    st = ctx.solve(nw.solver_cfg(kspace=30, max_iters=300, tol=tol, precond=nw.PREC_AMG,
+                                 mode=mode, inner_tol=1e-4))
+    n, nnz = tuple(ctx.amg_levels()[1])[:2]
+    assert 8 * n <= nnz <= 25 * n and (n >= 70000) == sliced, (n, nnz)
+    r = A.rhs - A.spmv(ctx.solution())
+    assert st.converged and np.linalg.norm(r) <= 1.0001 * tol * np.linalg.norm(A.rhs)
