@@ -177,6 +177,15 @@ __device__ inline SellLane sell_lane(bool stretch)
   return {(t / kWave) * R + lane % R, lane / R};
 }
 
+// Lanes that leave before the row sum: those without a row, or with several
+// lanes per row only whole waves of them (the others take part in its
+// butterfly).
+template <int G>
+__device__ inline bool sell_idle(SellLane l, int n)
+{
+  return (G == 1 ? l.row : l.row - l.row % (kWave / G)) >= n;
+}
+
 template <typename T, int G>
 __device__ inline T sell_dot(const SellView& A, const T* __restrict__ va,
                              const T* __restrict__ x, SellLane l, int n)
@@ -204,7 +213,8 @@ __device__ inline T sell_dot(const SellView& A, const T* __restrict__ va,
   const int base = A.base ? A.base[k] : -1;
   if (A.dia_w && A.dia_w[k] > 0) {
     const int32_t* off = A.dia_off + (int64_t)k * kDiaMax;
-    sum([&](int j) { return dia_column(row, off[j], n); });
+    // (the check of the row, 1 % of the product, only where lanes stay)
+    sum([&](int j) { return G == 1 ? row + off[j] : dia_column(row, off[j], n); });
   } else if (base >= 0) {
     sum([&](int j) { return base + A.cd[b + 64 * (int64_t)j]; });
   } else {
@@ -231,7 +241,7 @@ __global__ __launch_bounds__(kBlock) void k_sell_spmv(
   T alpha)
 {
   const SellLane l = sell_lane<G>(A.stretch);
-  if (l.row - l.row % (kWave / G) >= n) return;  // whole waves
+  if (sell_idle<G>(l, n)) return;
   const T s = sell_dot<T, G>(A, va, x, l, n);
   if (l.row < n && l.g == 0) y[l.row] = alpha * s;
 }
@@ -242,7 +252,7 @@ __global__ __launch_bounds__(kBlock) void k_sell_spmv_add(
   SellView A, const T* __restrict__ va, const T* __restrict__ x, T* __restrict__ y, int n)
 {
   const SellLane l = sell_lane<G>(A.stretch);
-  if (l.row - l.row % (kWave / G) >= n) return;
+  if (sell_idle<G>(l, n)) return;
   const T s = sell_dot<T, G>(A, va, x, l, n);
   if (l.row < n && l.g == 0) y[l.row] += s;
 }
@@ -271,7 +281,7 @@ __global__ __launch_bounds__(kBlock) void k_sell_smooth(
 {
   const SellLane l = sell_lane<G>(A.stretch);
   const int row = l.row;
-  if (row - row % (kWave / G) >= n) return;
+  if (sell_idle<G>(l, n)) return;
   const T s = sell_dot<T, G>(A, va, v, l, n);
   if (row < n && l.g == 0) {
     const T e = alpha * v[row] - beta * s;
@@ -286,7 +296,7 @@ __global__ __launch_bounds__(kBlock) void k_sell_resid(
   T* __restrict__ r, int n)
 {
   const SellLane l = sell_lane<G>(A.stretch);
-  if (l.row - l.row % (kWave / G) >= n) return;
+  if (sell_idle<G>(l, n)) return;
   const T s = sell_dot<T, G>(A, va, x, l, n);
   if (l.row < n && l.g == 0) r[l.row] = b[l.row] - s;
 }
