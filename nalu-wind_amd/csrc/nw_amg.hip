@@ -117,6 +117,11 @@ constexpr double kSellMaxAvgRow = 25.0;
 // 194.5, 90 204 / 209, 114 231 / 240, 132 248 / 262, 161 279 / 295, 189 306 /
 // 328; FP32 from equal at 77 to 215 / 232 at 161.
 constexpr int64_t kSellMinRows = 70000;
+// ... and, with fewer rows than hide it, no row of more than this many
+// entries, the walk of two lanes over which the launch ends with (the
+// restriction to 189 thousand rows of 15, the longest of 219, FP32: 23.4 us,
+// in CSR 21.1; restrictions to level 1 have 39 to 54 at most)
+constexpr int64_t kSellMaxRow = 128, kSellLongRows = 200000;
 
 template <typename T>
 static void mat_spmv(const DevMat<T>& M, const T* x, T* y, T alpha,
@@ -423,11 +428,11 @@ static int device_lmax(int n, double* x, double* y, const double* dinv, const M&
 }
 
 // Uploads a host CSR matrix.  Rows of more than kSellMaxAvgRow entries on
-// average, or fewer rows than kSellMinRows, stay in CSR: G lanes per row, that
-// take its average length at once, or four times that if the rows are ragged
-// (P and R: the longest has ten times the average; a level's own matrix is
-// slower with more lanes, 8.0 -> 10.3 us at twice as many for 43.5 thousand
-// rows of 28).  Others are packed into sliced ELL on the device from the
+// average, fewer rows than kSellMinRows, or few with long ones among them
+// stay in CSR: G lanes per row, that take its average length at once, or four
+// times that if the rows are ragged (P and R: the longest has ten times the
+// average; a level's own matrix is slower with more lanes, 8.0 -> 10.3 us at
+// twice as many for 43.5 thousand rows of 28).  Others are packed into sliced ELL on the device from the
 // uploaded CSR, with padding positions repeating the row's last column (value
 // 0), so that they stay inside the columns of a rectangular P or R.
 static int upload_mat(const amg::Csr& h, DevMat<double>& d, bool ragged, hipStream_t st)
@@ -438,7 +443,10 @@ static int upload_mat(const amg::Csr& h, DevMat<double>& d, bool ragged, hipStre
   const double avg = (double)nnz / (double)n;
   const std::vector<int32_t> rp(h.rp.begin(), h.rp.end());
   d.n = (int)n;
-  if (avg > kSellMaxAvgRow || n < kSellMinRows) {
+  bool long_rows = false;
+  if (n < kSellLongRows)
+    for (int64_t i = 0; i < n; ++i) long_rows |= rp[i + 1] - rp[i] > kSellMaxRow;
+  if (avg > kSellMaxAvgRow || n < kSellMinRows || long_rows) {
     d.G = lanes_per_row(ragged ? 4.0 * avg : avg);
     d.nv = nnz;
     NW_HIP(hipMalloc(&d.own_rp, sizeof(int32_t) * rp.size()));
