@@ -101,13 +101,15 @@ __device__ inline double mean_product(double a, double b, double c, double d)
 // FP64 divisions (about fifteen instructions each) are kept to those that the
 // formulas need per edge: uniform divisors (relaxation, time scale) come as
 // reciprocals from the host, those of a node are in derive().  Momentum had
-// ten per edge end and has one, continuity twelve and has two.  Measured with
-// the common body: momentum 128^3 0.60 -> 0.535 ms (its registers now hold
-// one slot in flight per lane without spilling; two spill and take 0.745),
-// one pass with the Peclet factor 61 x 127 x 45 103 -> 85 us, continuity
-// 192^3 0.730 -> 0.705 ms, mixed 96^3 220 -> 212 us: continuity is bound by
-// its L1 misses (58 M lines of 128 bytes a launch at 192^3, 66 in flight per
-// CU at any time), not by arithmetic, occupancy or loads in flight.
+// ten per edge end and has one, continuity twelve and has two.  Measured over
+// three meshes in turn, before and after the common body: momentum 128^3 with
+// its Peclet launch 621 -> 607 us (the kernel's registers hold one slot in
+// flight per lane without spilling; two spill and take 745 us), one pass with
+// the Peclet factor 61 x 127 x 45 100 -> 93 us (85 with the mesh in cache,
+// 103 before).  Continuity did not change (192^3 706 and 709 us, mixed 96^3
+// 208 and 208): it is bound by its L1 misses (58 M lines of 128 bytes a launch
+// at 192^3, 66 in flight per CU at any time), not by arithmetic, occupancy or
+// loads in flight.
 
 // s, m: buoyancy_source and its mask, loaded only with the balanced
 // buoyancy force (unused registers are dropped otherwise)
@@ -355,9 +357,9 @@ template <bool PEC>
 struct MomentumPhysT {
   static constexpr int NDOF = 3;
   static constexpr int kLanes = 2, kUnroll = 1, kUnroll2 = 1, kMinWaves = 2;
-  // persistent: 0.577 vs 0.643 ms on the 128^3 box; with the Peclet factor
-  // in the kernel (18 dwords of spill, 33 persistent) it is slower (0.95 vs
-  // 0.76 ms per step)
+  // persistent, with the Peclet launch: 607 vs 630 us on the 128^3 box.  The
+  // one-pass kernel is not: it was slower with two slots in flight, where it
+  // spilled; with one it would gain (89 vs 93 us on 61 x 127 x 45)
   static constexpr bool kNonTemporal = true, kPersistent = !PEC;
   // 32 rows of 7 slots (Hex8 edge graph); 72 bytes per slot of LDS
   static constexpr int kSlotsSmall = 224, kSlotsLarge = 224;

@@ -152,6 +152,12 @@ def test_what_leaves_one_end_of_an_edge_enters_the_other(nw, ctx):
     for kw in ({}, {"interp_together": 0.0}, {"incompressible": 1.0}):
         ctx.assemble_continuity(nw.continuity_defaults(**kw))
         opposite(1)
+    ctx.field_upload(nw.F_BUOYANCY_SOURCE, rng.normal(size=(2 * ne, 3)))
+    ctx.field_upload(nw.F_BUOYANCY_SOURCE_MASK, rng.uniform(0.0, 1.0, 2 * ne))
+    o = nw.continuity_defaults(balanced_buoyancy=1)
+    o.gravity[:] = [0.3, -0.2, -9.81]
+    ctx.assemble_continuity(o)
+    opposite(1)
     for limiter in (0, 1):
         s = nw.scalar_defaults(use_limiter=limiter, peclet=nw.Peclet(limiter, 1.0, 2.0, 4.0))
         ctx.assemble_scalar(s)
